@@ -39,6 +39,7 @@ SOURCES = [
     "quantize.hip",
     "sparsity.hip",
     "gemm_dense.hip",
+    "gemm_ring.hip",
     "gemm_skinny.hip",
     "gemm_decode.hip",
     "gemm_sparse.hip",

@@ -3,9 +3,9 @@
 // NHWC implicit GEMM (the MI355X form of config-5 shapes): output pixels are GEMM rows
 // (M = N*Ho*Wo), output channels GEMM columns, K = kH*kW*C in (kh, kw, c) order so
 // OHWI weights are already the (Co, K) row-major B operand. The A tile is gathered
-// straight from the NHWC image by ConvOperand (16 contiguous channels per chunk, zero
-// outside the padded image) into the same LDS-staged MFMA tile as the dense GEMM; no
-// im2col buffer is written. Integer sums do not depend on K order, so the INT32 stage
+// straight from the NHWC image (RingConv: 16 contiguous channels per chunk, zero outside the
+// padded image) into the same ring-fed MFMA tiles as the dense GEMM; no im2col buffer is
+// written. Integer sums do not depend on K order, so the INT32 stage
 // equals the reference's im2col GEMM (src/nn/int8_conv2d.cu:151-223, K order
 // ci*kH*kW + kh*kW + kw) on the same integers.
 //

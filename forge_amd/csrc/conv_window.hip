@@ -1,7 +1,7 @@
 // NHWC INT8 conv2d, stride 1, as a window-fed MFMA tile (configs[4]-class shapes: C % 128 == 0,
 // Co % 256 == 0, a few image rows per tile).
 //
-// The implicit GEMM of the dense engine (mfma_tile.h DmaConv) gathers a patch row per output
+// The implicit GEMM of the ring-fed tiles (ring_tile.h RingConv) gathers a patch row per output
 // pixel and tap, so a 3x3 conv moves every input byte through the LDS DMA nine times per tile.
 // Here a tile is R whole output rows of one image (TW = R * Wo = 32 NI pixels) x 256 output
 // channels: the input window those rows touch (R + (kH-1) dilH rows x Wo + (kW-1) dilW columns,
@@ -37,14 +37,6 @@ struct ConvWinArgs {
     int R, tiles_h;           // output rows per tile (32 NI pixels), tiles per image
     int tiles_m, tiles_n;     // row tiles, 256-channel column tiles
 };
-
-// s_waitcnt vmcnt(N) lgkmcnt(0) (expcnt unconstrained; gfx9 splits the 6-bit vmcnt over bits
-// [3:0] and [15:14]).
-template <int N>
-__device__ __forceinline__ void wait_vm_lgkm() {
-    static_assert(N >= 0 && N < 64, "vmcnt immediate");
-    __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4));
-}
 
 // Wave-uniform position of stage st = ch * T + tap.
 struct StagePos {
@@ -332,7 +324,7 @@ int launch_conv_window(const ConvGeom& g, const int8_t* w, const GemmEpilogue& e
 {
     const int N = g.rows / (g.Ho * g.Wo);
     const int kH = g.K / (g.C * g.kW), T = kH * g.kW;
-    if (g.strideH != 1 || g.strideW != 1 || g.C % kBK != 0 || Co % 256 != 0 || T < 2 || g.r0 != 0 ||
+    if (g.strideH != 1 || g.strideW != 1 || g.C % kBK != 0 || Co % 256 != 0 || T < 2 ||
         !ep.vec_out || ep.up_w != 0 || !aligned(g.x, 16) || !aligned(w, 16))
         return -1;
     const long long x_bytes = static_cast<long long>(N) * g.H * g.W * g.C;

@@ -23,6 +23,12 @@ int gemm_dense(const int8_t* A, const int8_t* B, const float* act_scale, const u
 // the upsample scatter, which the decode and skinny kernels do not implement.
 int gemm_tiles(const int8_t* A, const int8_t* B, const GemmEpilogue& ep, int M, int K, int N, hipStream_t s);
 
+// The ring-fed tiles (gemm_ring.hip): C = A (ep.M, K) x B (ep.N, K)^T with K % 16 == 0 and 16-byte
+// bases, every GemmEpilogue mode; and the NHWC conv gather with C % 16 == 0. -1 when an operand
+// is too large for its 32-bit offsets.
+int launch_ring_gemm(const int8_t* A, const int8_t* B, const GemmEpilogue& ep, int K, hipStream_t s);
+int launch_ring_conv(const ConvGeom& g, const int8_t* w, const GemmEpilogue& ep, hipStream_t s);
+
 // Skinny (M <= kSkinnyMaxM) weight-streaming GEMM; needs K % 16 == 0 and 16-byte bases.
 int launch_gemm_skinny(const int8_t* A, const int8_t* B, const GemmEpilogue& ep, int M, int K, int N,
                        hipStream_t s);

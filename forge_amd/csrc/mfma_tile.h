@@ -1,4 +1,5 @@
-// LDS-staged INT8 MFMA GEMM engines for gfx950 (v_mfma_i32_32x32x32_i8).
+// LDS-staged INT8 MFMA GEMM tile for gfx950 (v_mfma_i32_32x32x32_i8), and helpers shared by the
+// tile engines.
 //
 // One 256-thread workgroup (4 wavefronts in a 2 x 2 grid) computes a BM x BN INT32 tile of
 // C = A (rows, K) x B (cols, K)^T with both operands K-contiguous ("NT", the layout of the
@@ -15,25 +16,14 @@
 // offset 16*(l/32); both operands use the same (lane, byte) -> k assignment, so every
 // INT32 dot product is exact.
 //
-// Two K-loop engines share that layout and the epilogue:
-//
-// DmaTile (K % 128 == 0, 16-byte aligned row-major operands; the hot path): 128-byte K
-// stages in two LDS slots, filled by gfx950's LDS-DMA loads (buffer_load_dwordx4 ... lds
-// through a buffer resource per operand: each lane's 16 bytes land at M0 + 16*lane, no VGPR
-// staging, 32-bit offsets, the stage's K offset in the scalar offset). Every row of a stage is one full 128-byte
-// cache line read by 8 consecutive lanes; on gfx950 this sustains ~30 B/clk per CU into
-// LDS, against ~26 B/clk for 64-byte half-line rows, whatever the number of stages in
-// flight. Stage kt+1 streams in while stage kt is multiplied; MFMA fragments are read two
-// 32-deep sub-steps ahead of use into 4 register buffers, and the barrier that publishes
-// stage kt+1 sits in the middle of stage kt, so the LDS latency never reaches the MFMA
-// pipe. Synchronisation is explicit: one s_waitcnt vmcnt(0) lgkmcnt(0) (this wave's DMAs
-// landed, its reads of the old slot done) and one s_barrier per stage.
-// LDS rows are 8 chunks with the (r ^ (r >> 3)) & 7 swizzle below; the DMA lanes are
-// assigned (row, chunk) pairs so that each 1 KB DMA write lands exactly in that layout.
-//
-// NtTile (any K % 16 == 0 operand, including the implicit-im2col conv gather with zero
-// padding, and the byte-gather operands of odd shapes): 128-byte K stages through two LDS
-// buffers with one stage of register staging; rows of 8 chunks, swizzle (r ^ (r >> 3)) & 7.
+// NtTile (any operand: the implicit-im2col conv gather with zero padding, the byte-gather operands
+// of odd shapes, operands of 2 GiB and more): 128-byte K stages through two LDS buffers with one
+// stage of register staging; rows of 8 chunks, swizzle (r ^ (r >> 3)) & 7. 16-byte aligned
+// operands under 2 GiB run on the DMA-fed tiles of ring_tile.h, which share the LDS-DMA, wait and
+// swizzle helpers below. An LDS DMA (buffer_load_dwordx4 ... lds) lands each lane's 16 bytes at
+// M0 + 16 * lane with no VGPR staging; a CU sustains ~30 B/clk of it where every row of a stage
+// is one full 128-byte cache line read by 8 consecutive lanes, against ~26 B/clk for 64-byte
+// half-line rows, whatever the number of stages in flight.
 //
 // Edges: operand rows beyond the matrix are clamped to its last row (their products land in
 // accumulator entries that are never stored); the epilogue masks rows and columns.
@@ -56,6 +46,13 @@ template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
     static_assert(N >= 0 && N < 64, "vmcnt immediate");
     __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
+}
+
+// s_waitcnt vmcnt(N) lgkmcnt(0) (expcnt unconstrained).
+template <int N>
+__device__ __forceinline__ void wait_vm_lgkm() {
+    static_assert(N >= 0 && N < 64, "vmcnt immediate");
+    __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4));
 }
 
 // 16-byte global -> LDS DMA (global_load_lds_dwordx4): this lane's 16 bytes at `src` land at
@@ -164,7 +161,6 @@ struct ConvGeom {
     int K;      // kH * kW * C
     int H, W, C, Ho, Wo, kW;
     int padH, padW, strideH, strideW, dilH, dilW;
-    int r0 = 0; // operand row r is output pixel r0 + r (a launch over the rows from r0 on)
 };
 
 // Needs C % 16 == 0 (a chunk never straddles two taps) and a 16-byte aligned image.
@@ -327,206 +323,8 @@ struct NtTile {
     }
 };
 
-// ---- DMA engine (128-byte stages, 2-slot LDS ring, global_load_lds) ---------------------
-
 // s_waitcnt vmcnt(0) lgkmcnt(0) (expcnt unconstrained).
 __device__ __forceinline__ void wait_vm_lgkm0() { __builtin_amdgcn_s_waitcnt(0x7 << 4); }
-
-// DMA operand policies: where lane chunk c (16 bytes) of tile row r comes from at 128-deep
-// stage st. lane() runs once per DMA instruction; src() once per stage.
-
-// Row-major (rows, K) matrix, K % 128 == 0; rows past the end are clamped (never stored).
-// A row-major INT8 matrix as one buffer resource (rows * K < 2^31, checked by the host): a lane's
-// chunk offset is fixed, the stage's K offset is the uniform scalar offset of the buffer load,
-// so a stage's DMAs need no per-lane address arithmetic.
-struct DmaRowMajor {
-    const int8_t* p;
-    int rows, K;
-    using Lane = uint32_t;
-    __device__ __forceinline__ Lane lane(int r, int c) const {
-        return static_cast<uint32_t>(r < rows ? r : rows - 1) * static_cast<uint32_t>(K) + 16u * c;
-    }
-    using Stage = uint32_t;
-    __device__ __forceinline__ Stage stage(int st) const { return static_cast<uint32_t>(st) * kBK; }
-    __device__ __forceinline__ void dma(const Lane& l, Stage soff, int8_t* dst) const {
-        dma16_buf(buf_rsrc(p, static_cast<uint32_t>(rows) * static_cast<uint32_t>(K)), l, soff, dst);
-    }
-};
-
-// Implicit im2col of an NHWC image, K order (kh, kw, c): with C % 128 == 0 a 128-deep stage of a
-// patch row is one contiguous run of one input pixel's channels, or padding. The image is one
-// buffer resource (x_bytes < 2^31, set by the host with the magic multipliers), and a stage's
-// DMA is a buffer load at a 32-bit offset: the row's pixel offset (fixed per lane) plus the
-// stage's tap offset (uniform: (kh dilH W + kw dilW) C + c0). A row keeps a bit per tap saying
-// whether that tap lies inside the image; a padding tap gets an offset past the range, which
-// the hardware reads as zeros. Needs a 16-byte aligned image and kH kW <= 32.
-struct DmaConv : ConvGeom {
-    uint32_t x_bytes;            // bytes of the whole NHWC input
-    int cps;                     // 128-deep stages per tap (C / 128)
-    uint32_t mg_cps, mg_kw;      // udiv_magic multipliers for / cps and / kW
-    struct Lane {
-        int off;                 // byte offset of pixel (n, hb, wb) + 16 * chunk (may be negative)
-        uint32_t taps;           // bit kh kW + kw: tap inside the image
-    };
-    __device__ __forceinline__ Lane lane(int r, int c) const {
-        r += r0;
-        r = r < rows ? r : rows - 1;
-        const int wo = r % Wo;
-        const int t = r / Wo;
-        const int ho = t % Ho;
-        const int n = t / Ho;
-        const int hb = ho * strideH - padH, wb = wo * strideW - padW;
-        const int kH = K / (C * kW);
-        uint32_t taps = 0u;
-        for (int kh = 0; kh < kH; kh++)
-            for (int kw = 0; kw < kW; kw++) {
-                const int hi = hb + kh * dilH, wi = wb + kw * dilW;
-                if (hi >= 0 && hi < H && wi >= 0 && wi < W) taps |= 1u << (kh * kW + kw);
-            }
-        return Lane{((n * H + hb) * W + wb) * C + 16 * c, taps};
-    }
-    struct Stage {
-        int soff;                // (kh dilH W + kw dilW) C + c0
-        int tap;                 // kh kW + kw
-    };
-    __device__ __forceinline__ Stage stage(int st) const {
-        const int tap = udiv_magic(st, mg_cps), c0 = (st - tap * cps) * kBK;
-        const int kh = udiv_magic(tap, mg_kw), kw = tap - kh * kW;
-        return Stage{(kh * dilH * W + kw * dilW) * C + c0, tap};
-    }
-    __device__ __forceinline__ void dma(const Lane& l, const Stage& S, int8_t* dst) const {
-        const uint32_t voff = (l.taps >> S.tap) & 1u ? static_cast<uint32_t>(l.off + S.soff) : 0x80000000u;
-        dma16_buf(buf_rsrc(x, x_bytes), voff, 0, dst);
-    }
-};
-
-template <int BM, int BN>
-struct DmaTile {
-    static constexpr int kTM = BM / 2 / 32;
-    static constexpr int kTN = BN / 2 / 32;
-    static constexpr int kAIns = BM * (kBK / 16) / kWave / 4;   // 1 KB DMA instructions per wave per stage
-    static constexpr int kBIns = BN * (kBK / 16) / kWave / 4;
-    static constexpr int kSlotBytes = (BM + BN) * kBK;
-    static constexpr int kLdsBytes = 2 * kSlotBytes;
-    static_assert(kTM >= 1 && kTN >= 1 && kAIns >= 1 && kBIns >= 1, "tile too small");
-
-    // MFMA operand fragments of one 32-deep sub-step.
-    struct Frags {
-        v4i a[kTM];
-        v4i b[kTN];
-    };
-
-    v16i acc[kTN][kTM];
-
-    template <class OpA, class OpB>
-    __device__ __forceinline__ void run(const OpA& opa, const OpB& opb, int K, int m0, int n0, int8_t* lds) {
-        const int lane = threadIdx.x & (kWave - 1);
-        const int wave = threadIdx.x / kWave;
-        const int wm = (wave >> 1) * (BM / 2);
-        const int wn = (wave & 1) * (BN / 2);
-        const int l31 = lane & 31;
-        const int hi = lane >> 5;
-
-#pragma unroll
-        for (int j = 0; j < kTN; j++)
-#pragma unroll
-            for (int i = 0; i < kTM; i++)
-#pragma unroll
-                for (int e = 0; e < 16; e++) acc[j][i][e] = 0;
-
-        // DMA instruction q of this wave fills slot chunks s = (wave*kIns + q)*64 + lane:
-        // row s/8 (8 lanes read one 128-byte line), physical chunk s%8 = logical chunk
-        // (s%8) ^ swz(row) of that row.
-        typename OpA::Lane la[kAIns];
-        typename OpB::Lane lb[kBIns];
-#pragma unroll
-        for (int q = 0; q < kAIns; q++) {
-            const int s = (wave * kAIns + q) * kWave + lane;
-            const int r = s >> 3, c = (s & 7) ^ lds_swz8(r);
-            la[q] = opa.lane(m0 + r, c);
-        }
-#pragma unroll
-        for (int q = 0; q < kBIns; q++) {
-            const int s = (wave * kBIns + q) * kWave + lane;
-            const int r = s >> 3, c = (s & 7) ^ lds_swz8(r);
-            lb[q] = opb.lane(n0 + r, c);
-        }
-        const int nst = K / kBK;
-        // Stage st into slot st % 2; stages past the end re-read the last one (their slot is
-        // never read again), so the issue needs no branch.
-        auto issue = [&](int st) {
-            int8_t* slot = lds + (st & 1) * kSlotBytes;
-            const int sc = st < nst ? st : nst - 1;
-            const typename OpA::Stage sa = opa.stage(sc);
-            const typename OpB::Stage sb = opb.stage(sc);
-#pragma unroll
-            for (int q = 0; q < kAIns; q++) opa.dma(la[q], sa, slot + (wave * kAIns + q) * 1024);
-#pragma unroll
-            for (int q = 0; q < kBIns; q++) opb.dma(lb[q], sb, slot + BM * kBK + (wave * kBIns + q) * 1024);
-        };
-        auto load_frags = [&](int st, int ks, Frags& F) {
-            const int8_t* As = lds + (st & 1) * kSlotBytes;
-            const int8_t* Bs = As + BM * kBK;
-            const int c = 2 * ks + hi;
-#pragma unroll
-            for (int i = 0; i < kTM; i++)
-                F.a[i] = *reinterpret_cast<const v4i*>(As + lds_off128(wm + 32 * i + l31, c));
-#pragma unroll
-            for (int j = 0; j < kTN; j++)
-                F.b[j] = *reinterpret_cast<const v4i*>(Bs + lds_off128(wn + 32 * j + l31, c));
-        };
-        auto mfmas = [&](const Frags& F) {
-#pragma unroll
-            for (int j = 0; j < kTN; j++)
-#pragma unroll
-                for (int i = 0; i < kTM; i++)
-                    acc[j][i] = __builtin_amdgcn_mfma_i32_32x32x32_i8(F.b[j], F.a[i], acc[j][i], 0, 0, 0);
-        };
-        // Fragments are read two 32-deep sub-steps ahead of their MFMAs (4 register buffers,
-        // one rotation per stage), the reads and DMAs spread between the MFMAs (the scheduler
-        // would otherwise cluster them and expose the LDS latency). The barrier that
-        // publishes stage kt+1 sits after sub-step 1 of stage kt, once all of stage kt's
-        // reads are done, so sub-steps 2-3 can already read stage kt+1 and refill stage kt's
-        // slot with stage kt+2.
-        constexpr int kMf = kTM * kTN, kRd = kTM + kTN, kVm = (kAIns + kBIns) / 2;
-        Frags F0, F1, F2, F3;
-        issue(0);
-        wait_vm_lgkm0();
-        lds_barrier();
-        issue(1);
-        load_frags(0, 0, F0);
-        load_frags(0, 1, F1);
-        for (int kt = 0; kt + 1 < nst; kt++) {
-            load_frags(kt, 2, F2);
-            mfmas(F0);
-            sched_interleave<kMf, kRd, 0>();
-            load_frags(kt, 3, F3);
-            mfmas(F1);
-            sched_interleave<kMf, kRd, 0>();
-            // Stage kt+1 landed (own DMAs) and this wave's reads of stage kt are complete.
-            wait_vm_lgkm0();
-            lds_barrier();
-            issue(kt + 2);                         // into stage kt's slot
-            load_frags(kt + 1, 0, F0);
-            mfmas(F2);
-            load_frags(kt + 1, 1, F1);
-            mfmas(F3);
-            // The DMAs first (spread over sub-step 2), then the reads (over sub-step 3): a
-            // global_load_lds also matches the LDS-read group, so the two are not mixed.
-            sched_interleave<kMf, 0, 2 * kVm>();
-            sched_interleave<kMf, 2 * kRd, 0>();
-        }
-        load_frags(nst - 1, 2, F2);
-        mfmas(F0);
-        load_frags(nst - 1, 3, F3);
-        mfmas(F1);
-        mfmas(F2);
-        mfmas(F3);
-        // Every wave is done with the ring (and no DMA is in flight) before the epilogue.
-        wait_vm_lgkm0();
-        lds_barrier();
-    }
-};
 
 // ---- shared epilogue -------------------------------------------------------------------
 
@@ -822,8 +620,8 @@ __device__ __forceinline__ void store_tile(const v16i (&acc)[BN / 64][BM / 64], 
 // grid whose first id is not a multiple of 8 shifts which XCD gets which run, not the
 // grouping), then runs are rasterised in groups of kGroupM tile-rows: an XCD's L2 then
 // holds a few A row-blocks and B col-blocks instead of all of them.
+constexpr int kGroupM = 4;
 __device__ __forceinline__ void tile_coords(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
-    constexpr int kGroupM = 4;
     const int total = tiles_m * tiles_n;
     const int t = xcd_contiguous(bid, total);
     const int per_group = kGroupM * tiles_n;
