@@ -9,7 +9,8 @@
 // equals the reference's im2col GEMM (src/nn/int8_conv2d.cu:151-223, K order
 // ci*kH*kW + kh*kW + kw) on the same integers.
 //
-// NCHW FP16 API (src/nn/int8_conv2d.cu:126-223): per sample, the patch matrix
+// NCHW FP16 API (src/nn/int8_conv2d.cu:126-223): small layers in one launch (below), deep ones in
+// two (conv_deep.hip). What neither takes: per sample, the patch matrix
 // [Ho*Wo, C_in*kH*kW] is gathered to FP16 in the caller's workspace, quantized per patch
 // row, multiplied with the dequant epilogue, and transposed to NCHW -- the reference's
 // workspace contract (one sample's buffers) fixes that per-sample structure.
@@ -1186,6 +1187,20 @@ extern "C" int forge_int8_conv2d_forward(const uint16_t* input, const int8_t* we
         size_t lds = 0;
         if (conv_nchw_cl_plan(a, &lds, 8) || conv_nchw_cl_plan(a, &lds, 4)) return conv_nchw_cl(a, lds, s);
     }
+    const size_t ws_bytes = forge_int8_conv2d_workspace_size(C_in, H, W, C_out, kH, kW, padH, padW, strideH, strideW,
+                                                             dilH, dilW);
+    const ConvDeepShape deep{input, weight, w_scale, bias, output, N, C_in, H, W, C_out, kH, kW, padH, padW,
+                             strideH, strideW, dilH, dilW, Ho, Wo};
+    // From 48 input channels on, and 48 output channels or 4096 pairs, the NCHW-window kernel below
+    // reads its 16-tap chunks and weights too slowly (us, it / conv_deep: 144 -> 32 at 167 x 376
+    // 62 / 25, 64 -> 64 at 134 x 201 33 / 20, 96 -> 96 at 100 x 101 28 / 25, 128 -> 64 at 60 x 80
+    // 17.1 / 16.3); smaller layers (128 -> 32) and few pixels (80 -> 80, 340 pixels: 13.9 / 16.9) stay
+    // on it.
+    if (C_in >= 48 && (C_out >= 48 || static_cast<long long>(C_in) * C_out > 4096) &&
+        static_cast<long long>(N) * M >= 4096) {
+        const int r = launch_conv_deep(deep, workspace, ws_bytes, s);
+        if (r != -1) return r;
+    }
     {
         ConvNchwArgs a{input, weight, w_scale, bias, output, C_in, H, W, C_out, kH, kW, padH, padW, strideH, strideW,
                        dilH, dilW, Ho, Wo, K};
@@ -1210,6 +1225,10 @@ extern "C" int forge_int8_conv2d_forward(const uint16_t* input, const int8_t* we
             else conv_nchw_fused_kernel<false, false><<<grid, 256, lds, s>>>(a);
             return launch_status();
         }
+    }
+    {
+        const int r = launch_conv_deep(deep, workspace, ws_bytes, s);
+        if (r != -1) return r;
     }
     note_route("conv-nchw-per-image");
     auto up = [](size_t b) { return (b + 255) & ~static_cast<size_t>(255); };

@@ -99,6 +99,18 @@ int launch_sparse_wide_s32(const int8_t* W_comp, const int8_t* x, const uint32_t
 // returns -1 when the shape is not one it takes.
 int launch_conv_window(const ConvGeom& g, const int8_t* w, const GemmEpilogue& ep, int Co, hipStream_t s);
 
+// NCHW FP16 conv of deep layers (conv_deep.hip) in two launches per workspace-sized chunk of
+// images; returns -1 when the shape is not one it takes.
+struct ConvDeepShape {
+    const uint16_t* x;
+    const int8_t* w;
+    const uint16_t* w_scale;
+    const uint16_t* bias;
+    uint16_t* y;
+    int N, C, H, W, Co, kH, kW, padH, padW, sH, sW, dH, dW, Ho, Wo;
+};
+int launch_conv_deep(const ConvDeepShape& c, void* workspace, size_t ws_bytes, hipStream_t s);
+
 // Implicit-GEMM NHWC conv through the dense tile engine (conv.hip supplies the geometry).
 int launch_conv_gemm(const ConvGeom& g, const int8_t* w, const GemmEpilogue& ep, int Co, bool vec,
                      hipStream_t s);

@@ -300,3 +300,52 @@ def test_conv_nchw_fused_special_values(dev, orc, W, Co, route):
     y, got_route = _nchw_run(dev, x, w, ws, b, 3, 1, 1, 1)
     assert got_route == route, got_route
     _nchw_check(orc, y, x, w, ws, b, 3, 1, 1, 1)
+
+
+# "conv-nchw-deep": deep layers, 32-channel window chunks and streamed weights. 128 -> 128 (aligned
+# loads); C and C_out no multiples of 32 at an odd width (shifted end-of-row groups); two groups of
+# output channels at stride 2; 25 taps in three slots; 4 taps; dilation 2; 49 taps; a width of 8;
+# one output row per tile; enough tiles for several per CU.
+DEEP_CASES = [(3, 128, 20, 24, 136, 3, 1, 1, 1, True), (3, 80, 41, 35, 72, 3, 1, 1, 1, True),
+              (3, 96, 33, 40, 160, 3, 1, 2, 1, False), (3, 64, 14, 45, 96, 5, 2, 1, 1, True),
+              (3, 72, 41, 36, 64, 2, 0, 1, 1, True), (3, 64, 46, 31, 64, 3, 2, 1, 2, True),
+              (2, 64, 20, 36, 48, 7, 3, 1, 1, True), (4, 96, 40, 8, 160, 3, 1, 1, 1, True),
+              (2, 48, 6, 390, 200, 3, 1, 1, 1, False), (2, 64, 150, 203, 160, 3, 0, 1, 1, True),
+              (200, 64, 20, 20, 64, 3, 1, 2, 1, True)]   # channel maxima in two workspace-sized chunks
+
+
+@pytest.mark.parametrize("N,C,H,W,Co,k,pad,stride,dil,bias", DEEP_CASES)
+def test_conv_nchw_deep(dev, orc, N, C, H, W, Co, k, pad, stride, dil, bias):
+    rng = np.random.default_rng(C * W + Co + k + 1)
+    x = rng.uniform(-1, 1, (N, C, H, W)).astype(np.float16)
+    w = int8_uniform(rng, (Co, C * k * k))
+    ws = rng.uniform(0.005, 0.05, Co).astype(np.float16)
+    b = rng.uniform(-0.5, 0.5, Co).astype(np.float16) if bias else None
+    say(f"conv nchw deep N={N} C={C} H={H} W={W} Co={Co} k={k} s={stride} d={dil}")
+    y, route = _nchw_run(dev, x, w, ws, b, k, pad, stride, dil)
+    assert route.startswith("conv-nchw-deep"), route
+    _nchw_check(orc, y, x, w, ws, b, k, pad, stride, dil)
+
+
+@pytest.mark.parametrize("W", [80, 83])
+def test_conv_nchw_deep_special_values(dev, orc, W):
+    """NaN, +-inf, subnormal and all-zero windows, an input one element past an aligned start."""
+    import torch
+    from forge_amd import ops
+    from helpers import special_fp16_rows
+    rng = np.random.default_rng(78)
+    N, C, H, Co = 2, 64, 27, 160
+    x = special_fp16_rows(rng, N * C * H, W).reshape(N, C, H, W)
+    x[1, :, 4:7, 10:20] = 0
+    w = int8_uniform(rng, (Co, C * 9))
+    ws = rng.uniform(0.005, 0.05, Co).astype(np.float16)
+    b = rng.uniform(-0.5, 0.5, Co).astype(np.float16)
+    say(f"conv nchw deep special values W={W}")
+    y, route = _nchw_run(dev, x, w, ws, b, 3, 1, 1, 1)
+    assert route.startswith("conv-nchw-deep"), route
+    _nchw_check(orc, y, x, w, ws, b, 3, 1, 1, 1)
+    buf = torch.empty((x.size + 1,), dtype=torch.float16, device=dev)
+    buf[1:].copy_(to_dev(x, dev).view(-1))
+    y1 = to_host(ops.int8_conv2d_forward(buf[1:].view(N, C, H, W), to_dev(w, dev), to_dev(ws, dev), to_dev(b, dev), 3, 3,
+                                         (1, 1)))
+    assert np.array_equal(y1.view(np.uint16), y.view(np.uint16))
