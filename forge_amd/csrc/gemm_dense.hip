@@ -132,6 +132,11 @@ int launch_conv_gemm(const ConvGeom& g, const int8_t* w, const GemmEpilogue& ep,
     }
     ConvBytes a;
     static_cast<ConvGeom&>(a) = g;
+    if (K < 16) {
+        RowMajorShort b{w, Co, K};
+        return ep.c16 ? dispatch_tiles<false, true, false>(a, b, ep, M, Co, K, s)
+                      : dispatch_tiles<false, false, false>(a, b, ep, M, Co, K, s);
+    }
     RowMajorBytes b{w, Co, K};
     return ep.c16 ? dispatch_tiles<false, true, false>(a, b, ep, M, Co, K, s)
                   : dispatch_tiles<false, false, false>(a, b, ep, M, Co, K, s);
@@ -181,6 +186,11 @@ int gemm_tiles(const int8_t* A, const int8_t* B, const GemmEpilogue& ep, int M, 
         RowMajorOperand a{A, M, K}, b{B, N, K};
         const bool even = K % kBK == 0;
         return out16 ? dispatch_k<true>(a, b, ep, M, N, K, even, s) : dispatch_k<false>(a, b, ep, M, N, K, even, s);
+    }
+    if (K < 16) {
+        RowMajorShort a{A, M, K}, b{B, N, K};
+        return out16 ? dispatch_tiles<false, true, false>(a, b, ep, M, N, K, s)
+                     : dispatch_tiles<false, false, false>(a, b, ep, M, N, K, s);
     }
     RowMajorBytes a{A, M, K}, b{B, N, K};
     return out16 ? dispatch_tiles<false, true, false>(a, b, ep, M, N, K, s)

@@ -19,8 +19,34 @@
 
 namespace forge_amd {
 
-// One 256-thread workgroup per row; K % 8 == 0, K <= VPT * 2048, x 16-byte and q 8-byte
-// aligned. Thread t holds 16-byte vectors t, t + 256, ... of its row in VGPRs (x is read
+// A row as vectors of 8 values (16 bytes of x, 8 of q). ALIGNED: K % 8 == 0, x 16-byte and q 8-byte
+// aligned. Otherwise any K >= 8 at the element alignment (gfx950 loads and stores vectors at any
+// address), the last vector moved back to end with the row: it overlaps the one before, whose
+// values it reads, quantizes and writes once more the same.
+template <bool ALIGNED>
+struct RowVecs {
+    const uint16_t* src;
+    int8_t* dst;
+    int K, nvec;
+    __device__ __forceinline__ RowVecs(const uint16_t* x, int8_t* q, int row, int K_)
+        : src(x + static_cast<size_t>(row) * K_), dst(q + static_cast<size_t>(row) * K_), K(K_), nvec((K_ + 7) >> 3) {}
+    __device__ __forceinline__ uint4 load(int i) const {
+        if constexpr (ALIGNED) return reinterpret_cast<const uint4*>(src)[i];
+        typedef uint32_t u4 __attribute__((ext_vector_type(4), aligned(2)));
+        const u4 v = *reinterpret_cast<const u4*>(src + min(8 * i, K - 8));
+        return make_uint4(v[0], v[1], v[2], v[3]);
+    }
+    __device__ __forceinline__ void store(int i, uint2 v) const {
+        if constexpr (ALIGNED) {
+            reinterpret_cast<uint2*>(dst)[i] = v;
+            return;
+        }
+        typedef uint32_t u2 __attribute__((ext_vector_type(2), aligned(1)));
+        *reinterpret_cast<u2*>(dst + min(8 * i, K - 8)) = u2{v.x, v.y};
+    }
+};
+
+// One 256-thread workgroup per row; K <= VPT * 2048. Thread t holds 16-byte vectors t, t + 256, ... of its row in VGPRs (x is read
 // once) and every lane writes 8 int8 per vector. Spreading a row over 4 waves keeps
 // decode-size calls (a handful of rows) from serialising one wave's loads.
 //
@@ -31,7 +57,7 @@ namespace forge_amd {
 // DPP across the wave, 4 entries through LDS); a row holding a NaN takes the fp32 maximum,
 // which skips NaN as fmaxf does. Values are quantized by quant8_row, bit-equal to quant8
 // for a row's own scale.
-template <int VPT>
+template <int VPT, bool ALIGNED = true>
 __global__ __launch_bounds__(256) void quantize_rows_block_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q, float* __restrict__ scales, int K)
 {
@@ -39,12 +65,11 @@ __global__ __launch_bounds__(256) void quantize_rows_block_kernel(
     __shared__ float wmax[4];
     const int row = blockIdx.x;
     const int t = threadIdx.x, lane = t & (kWave - 1), wave = t / kWave;
-    const int nvec = K >> 3;
-    const uint4* src = reinterpret_cast<const uint4*>(x + static_cast<size_t>(row) * K);
-    uint2* dst = reinterpret_cast<uint2*>(q + static_cast<size_t>(row) * K);
+    const RowVecs<ALIGNED> rv(x, q, row, K);
+    const int nvec = rv.nvec;
     uint4 v[VPT];
 #pragma unroll
-    for (int i = 0; i < VPT; i++) v[i] = src[min(t + i * 256, nvec - 1)];
+    for (int i = 0; i < VPT; i++) v[i] = rv.load(min(t + i * 256, nvec - 1));
     uint32_t m = 0u;
 #pragma unroll
     for (int i = 0; i < VPT; i++) m = absbits8(v[i], m);
@@ -70,7 +95,7 @@ __global__ __launch_bounds__(256) void quantize_rows_block_kernel(
 #pragma unroll
     for (int i = 0; i < VPT; i++) {
         const int idx = t + i * 256;
-        if (idx < nvec) dst[idx] = quant8_row(v[i], inv);
+        if (idx < nvec) rv.store(idx, quant8_row(v[i], inv));
     }
 }
 
@@ -80,19 +105,18 @@ __global__ __launch_bounds__(256) void quantize_rows_block_kernel(
 // 6.06 TB/s of 50.3 MB). Lane t holds vectors t, t + 64,
 // ... of its row; loads, absmax and quantization as in the kernel above, the absmax reduced
 // within the wave by DPP.
-template <int VPT>
+template <int VPT, bool ALIGNED = true>
 __global__ __launch_bounds__(256) void quantize_rows_wave_kernel(
     const uint16_t* __restrict__ x, int8_t* __restrict__ q, float* __restrict__ scales, int M, int K)
 {
     const int lane = threadIdx.x & (kWave - 1);
     const int row = blockIdx.x * 4 + static_cast<int>(threadIdx.x / kWave);
     if (row >= M) return;                    // whole waves leave: the DPP reduction sees 64 lanes
-    const int nvec = K >> 3;
-    const uint4* src = reinterpret_cast<const uint4*>(x + static_cast<size_t>(row) * K);
-    uint2* dst = reinterpret_cast<uint2*>(q + static_cast<size_t>(row) * K);
+    const RowVecs<ALIGNED> rv(x, q, row, K);
+    const int nvec = rv.nvec;
     uint4 v[VPT];
 #pragma unroll
-    for (int i = 0; i < VPT; i++) v[i] = src[min(lane + i * kWave, nvec - 1)];
+    for (int i = 0; i < VPT; i++) v[i] = rv.load(min(lane + i * kWave, nvec - 1));
     uint32_t m = 0u;
 #pragma unroll
     for (int i = 0; i < VPT; i++) m = absbits8(v[i], m);
@@ -112,7 +136,7 @@ __global__ __launch_bounds__(256) void quantize_rows_wave_kernel(
 #pragma unroll
     for (int i = 0; i < VPT; i++) {
         const int idx = lane + i * kWave;
-        if (idx < nvec) dst[idx] = quant8_row(v[i], inv);
+        if (idx < nvec) rv.store(idx, quant8_row(v[i], inv));
     }
 }
 
@@ -307,29 +331,36 @@ namespace forge_amd {
 // small and a whole workgroup per row spreads each row's loads wider.
 constexpr int kWaveRowsMinM = 2048;
 
-int launch_quantize(const uint16_t* x, int8_t* q, float* scales, int M, int K, hipStream_t s)
+template <bool ALIGNED>
+static int launch_quantize_rows(const uint16_t* x, int8_t* q, float* scales, int M, int K, hipStream_t s)
 {
-    const bool vec_ok = (K % 8 == 0) && K <= 8 * 2048 && aligned(x, 16) && aligned(q, 8);
-    if (vec_ok && K <= 4096 && M >= kWaveRowsMinM) {
+    if (K <= 4096 && M >= kWaveRowsMinM) {
         const int vpt = divup(K, 8 * kWave);
         const unsigned grid = static_cast<unsigned>(divup(M, 4));
-        if (vpt <= 1)      quantize_rows_wave_kernel<1><<<grid, 256, 0, s>>>(x, q, scales, M, K);
-        else if (vpt <= 2) quantize_rows_wave_kernel<2><<<grid, 256, 0, s>>>(x, q, scales, M, K);
-        else if (vpt <= 4) quantize_rows_wave_kernel<4><<<grid, 256, 0, s>>>(x, q, scales, M, K);
-        else               quantize_rows_wave_kernel<8><<<grid, 256, 0, s>>>(x, q, scales, M, K);
+        if (vpt <= 1)      quantize_rows_wave_kernel<1, ALIGNED><<<grid, 256, 0, s>>>(x, q, scales, M, K);
+        else if (vpt <= 2) quantize_rows_wave_kernel<2, ALIGNED><<<grid, 256, 0, s>>>(x, q, scales, M, K);
+        else if (vpt <= 4) quantize_rows_wave_kernel<4, ALIGNED><<<grid, 256, 0, s>>>(x, q, scales, M, K);
+        else               quantize_rows_wave_kernel<8, ALIGNED><<<grid, 256, 0, s>>>(x, q, scales, M, K);
         return launch_status();
     }
-    if (vec_ok) {
-        const int vpt = divup(K, 2048);
-        if (vpt <= 1)      quantize_rows_block_kernel<1><<<M, 256, 0, s>>>(x, q, scales, K);
-        else if (vpt <= 2) quantize_rows_block_kernel<2><<<M, 256, 0, s>>>(x, q, scales, K);
-        else if (vpt <= 4) quantize_rows_block_kernel<4><<<M, 256, 0, s>>>(x, q, scales, K);
-        else               quantize_rows_block_kernel<8><<<M, 256, 0, s>>>(x, q, scales, K);
-    } else {
+    const int vpt = divup(K, 2048);
+    if (vpt <= 1)      quantize_rows_block_kernel<1, ALIGNED><<<M, 256, 0, s>>>(x, q, scales, K);
+    else if (vpt <= 2) quantize_rows_block_kernel<2, ALIGNED><<<M, 256, 0, s>>>(x, q, scales, K);
+    else if (vpt <= 4) quantize_rows_block_kernel<4, ALIGNED><<<M, 256, 0, s>>>(x, q, scales, K);
+    else               quantize_rows_block_kernel<8, ALIGNED><<<M, 256, 0, s>>>(x, q, scales, K);
+    return launch_status();
+}
+
+int launch_quantize(const uint16_t* x, int8_t* q, float* scales, int M, int K, hipStream_t s)
+{
+    // Rows under 8 values, and those past the registers, take the two-pass kernel.
+    if (K < 8 || K > 8 * 2048) {
         forge::quant::fused_quantize_activation_kernel<<<M, 256, 0, s>>>(
             reinterpret_cast<const __half*>(x), q, scales, K);
+        return launch_status();
     }
-    return launch_status();
+    if (K % 8 == 0 && aligned(x, 16) && aligned(q, 8)) return launch_quantize_rows<true>(x, q, scales, M, K, s);
+    return launch_quantize_rows<false>(x, q, scales, M, K, s);
 }
 
 int launch_quantize_pixels_nchw(const uint16_t* x, int8_t* q, float* scales, int images, int C, int HW,
