@@ -36,6 +36,7 @@ SIGNATURES = {
     "forge_int8_gemm": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _P]),
     "forge_int8_linear": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _P, _P, _P]),
     "forge_int8_gemm_s32": (_I, [_P, _P, _P, _I, _I, _I, _P]),
+    "forge_int8_linear_backward_prep": (_I, [_P, _P, _P, _P, _P, _P, _I, _I, _I, _P]),
     "forge_int8_linear_noalloc": (_I, [_P, _P, _P, _P, _P, _I, _I, _I, _P]),
     "forge_prune_compress_24": (_I, [_P, _P, _P, _I, _I, _P]),
     "forge_pack_metadata": (_I, [_P, _P, _I, _I, _P]),

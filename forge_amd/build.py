@@ -49,6 +49,7 @@ SOURCES = [
     "conv_window.hip",
     "conv_transpose.hip",
     "conv_depthwise.hip",
+    "linear_backward.hip",
     "noalloc.hip",
     "forge_api.cpp",
 ]

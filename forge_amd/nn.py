@@ -50,7 +50,15 @@ class _Int8LinearFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_output):
         w_int8, w_scale = ctx.saved_tensors
-        g = grad_output.to(torch.float16)
+        g = grad_output if grad_output.dtype == torch.float16 else grad_output.to(torch.float16)
+        # With gradients recorded (create_graph=True) the torch operators below carry them; the
+        # library's passes would not. It sums whole FP16 vectors of a non-empty batch.
+        if (not torch.is_grad_enabled() and grad_output.dtype == torch.float16 and g.is_cuda and w_int8.is_cuda
+                and w_int8.is_contiguous() and w_scale.dtype == torch.float16 and g.shape[0] > 0 and g.shape[1] >= 8):
+            if not g.is_contiguous():
+                g = g.contiguous()
+            w16, grad_bias = ops.int8_linear_backward_prep(w_int8, w_scale, g, ctx.has_bias)
+            return g @ w16, None, None, grad_bias, None, None
         w16 = w_int8.to(torch.float16) * w_scale.unsqueeze(1)
         grad_x = g @ w16
         grad_bias = grad_output.sum(dim=0).to(torch.float16) if ctx.has_bias else None

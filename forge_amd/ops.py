@@ -200,6 +200,26 @@ def int8_gemm_s32(A: torch.Tensor, B: torch.Tensor, out: Optional[torch.Tensor] 
     return out
 
 
+COLUMN_SUM_PARTS = 32   # FORGE_COLUMN_SUM_PARTS
+
+
+def int8_linear_backward_prep(w_int8: torch.Tensor, w_scale: torch.Tensor, grad: torch.Tensor, has_bias: bool):
+    """What int8_linear's input gradient multiplies grad (M, N) with, the FP16 weight as an (N, K)
+    tensor contiguous along N, and the bias gradient (N,) or None (N >= 8)."""
+    N, K = w_int8.shape
+    _need(w_int8, torch.int8, "w_int8")
+    _need(w_scale, torch.float16, "w_scale", N)
+    _need(grad, torch.float16, "grad")
+    w16 = torch.empty_strided((N, K), (1, N), dtype=torch.float16, device=grad.device)
+    partial = grad_bias = None
+    if has_bias:
+        partial = torch.empty((COLUMN_SUM_PARTS, N), dtype=torch.float32, device=grad.device)
+        grad_bias = torch.empty((N,), dtype=torch.float16, device=grad.device)
+    _call("forge_int8_linear_backward_prep", _p(w_int8), _p(w_scale), _p(w16), _p(grad), _p(partial), _p(grad_bias),
+          grad.shape[0], K, N, _stream())
+    return w16, grad_bias
+
+
 # ---- sparsity (bindings.cpp:558-575) ------------------------------------------------
 
 def prune_compress_24(weight: torch.Tensor, compressed: torch.Tensor, metadata_raw: torch.Tensor,

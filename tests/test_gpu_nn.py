@@ -8,7 +8,7 @@ dequantized FP16 weight), and the w_meta conversion to and from the reference's 
 import numpy as np
 import pytest
 
-from helpers import fp16_normal, say, to_dev, to_host
+from helpers import fp16_normal, int8_uniform, say, to_dev, to_host
 
 pytestmark = pytest.mark.gpu
 
@@ -64,6 +64,38 @@ def test_quantized_linear_backward(dev):
     assert x.grad.shape == (M, K) and x.grad.dtype == torch.float16
     assert torch.allclose(x.grad.float().cpu(), gx_ref, rtol=2e-2, atol=2e-2)
     assert torch.allclose(m.bias.grad.float().cpu(), g.float().sum(0).cpu(), rtol=1e-2, atol=1e-2)
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 16, 8), (17, 100, 70), (513, 588, 1001), (2048, 256, 512), (70, 64, 65), (40, 20, 3)])
+def test_linear_backward_passes(dev, M, K, N):
+    """The backward's own kernels at ragged sizes. The FP16 weight has the bits of the torch
+    expression; the column sums, in FP32 over M terms, are within M 2^-24 sum|g| of the FP64 ones
+    before the rounding to FP16 (half an ulp, 2^-11); the gradients equal those through the torch
+    operators (taken with create_graph) to the FP16 rounding of a sum in another order."""
+    import torch
+    from forge_amd import ops
+    from forge_amd.nn import QuantizedLinear
+    rng = np.random.default_rng(M + K + N)
+    w = to_dev(int8_uniform(rng, (N, K)), dev)
+    ws = to_dev(rng.uniform(1e-3, 1e-2, N).astype(np.float16), dev)
+    g = to_dev(fp16_normal(rng, (M, N)), dev)
+    say(f"linear backward passes M={M} K={K} N={N}")
+    want = (w.to(torch.float16) * ws.unsqueeze(1)).t().contiguous()
+    w16, gb = ops.int8_linear_backward_prep(w, ws, g, N >= 8)
+    assert np.array_equal(to_host(w16.t()).view(np.uint16), to_host(want).view(np.uint16))
+    if N >= 8:
+        ref, bound = g.double().sum(0), g.double().abs().sum(0) * (M * 2.0 ** -24)
+        err = (gb.double() - ref).abs()
+        assert bool((err <= bound + (ref.abs() + bound) * 2.0 ** -11 + 2.0 ** -25).all())
+    m = QuantizedLinear(K, N).to(dev)
+    m.w_int8.copy_(w)
+    m.w_scale.data.copy_(ws)
+    x = to_dev(fp16_normal(rng, (M, K)), dev).requires_grad_(True)
+    gx, gb = torch.autograd.grad(m(x), (x, m.bias), g)
+    gx2, gb2 = torch.autograd.grad(m(x), (x, m.bias), g, create_graph=True)
+    scale = float((g.float().abs() @ want.float().abs().t()).max())
+    assert float((gx.float() - gx2.float()).abs().max()) <= scale * (N * 2.0 ** -24 + 2.0 ** -10)
+    assert float((gb.float() - gb2.float()).abs().max()) <= float(g.float().abs().sum(0).max()) * (M * 2.0 ** -24 + 2.0 ** -10)
 
 
 @pytest.mark.parametrize("M,K,N,bias", [(5, 256, 64, True), (200, 1280, 320, True), (129, 512, 96, False)])
