@@ -4,8 +4,8 @@
 // pixel owns one 2x2 output block, so the layer is a GEMM of the per-pixel quantized input
 // rows (H*W, C_in) with the repacked weights (4*C_out, C_in), row co*4 + kh*2 + kw, followed
 // by a scatter to NCHW. The reference runs transpose -> quantize -> GEMM to an FP16 buffer
-// -> scatter + bias, one image at a time. Here, for C_in in {32, 64, 128, 256} and
-// H*W % 8 == 0, convt_fused_kernel does all of it in one pass per 32-pixel tile (described at
+// -> scatter + bias, one image at a time. Here, for C_in a multiple of 32 up to 256
+// and H*W % 8 == 0, convt_fused_kernel does all of it in one pass per 32-pixel tile (described at
 // the kernel): input read once, INT8 activations kept in LDS, output written once, one launch
 // for all images, no workspace traffic. Every other shape takes two kernels:
 //   1. quantize_pixels_nchw reads the NCHW image once and writes the INT8 pixel rows and
@@ -29,7 +29,7 @@ namespace forge_amd {
 
 static size_t up256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
 
-// Single-pass kernel for C_in = 32 * KC (KC = 1, 2, 4, 8), H*W % 8 == 0: one workgroup (2 waves)
+// Single-pass kernel for C_in = 32 * KC (KC = 1 .. 8), H*W % 8 == 0: one workgroup (2 waves)
 // takes 32 consecutive pixels of one image and writes their whole (C_out, 2x2) output, so the
 // INT8 activations never leave the chip and the input is read once. Tiles of 32 pixels (one MFMA
 // row block) rather than 64 give twice the workgroups, whose load, compute and store phases then
@@ -42,7 +42,7 @@ static size_t up256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
 //      then over the wave's 16 channel groups (lane shuffles) and the 2 waves (LDS): the row
 //      arithmetic of quantize_rows on each pixel's C_in values.
 //   2. The quantized pixels form the A tile in LDS (32 x C_in bytes, 16-byte chunks swizzled
-//      by row so the MFMA row reads spread over the banks).
+//      by row, or rows padded, so the MFMA row reads spread over the banks).
 //   3. Work items (n-block j of 32 GEMM columns for the tile's 32 pixels) go round-robin to the
 //      2 waves; B fragments are the weight rows, read from L2 straight into registers; K is
 //      KC steps of v_mfma_i32_32x32x32_i8.
@@ -55,6 +55,9 @@ static size_t up256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
 // 16 accumulators in VGPRs beside the rest (67 at C_in = 64, 7 waves; 86 registers and 5 waves
 // otherwise), (1,64,270,480)->32 20.5 -> 19.0-19.1 us, (1,32,540,960)->16 33 -> 29.7-30.3 us. At 128
 // and 256 channels that limit spills, so those keep the default.
+// Channel counts between the powers of two, against the two-kernel path they took (quantize_pixels_
+// nchw, then the GEMM with the scatter): (2,96,180,320) -> 48 54.3 -> 22.6 us, (2,160,193,152) -> 80
+// 56.6 -> 22.9, (1,192,135,240) -> 96 35.4 -> 18.5, (1,224,80,160) -> 64 17.8 -> 10.3.
 template <int KC>
 constexpr int convt_min_waves() { return KC <= 2 ? 6 : 1; }
 
@@ -69,8 +72,12 @@ __global__ __launch_bounds__(128, convt_min_waves<KC>()) void convt_fused_kernel
     constexpr int kNW = PT / 16;                     // waves: 4 * PT threads
     constexpr int kPG = PT / 8;                      // 8-pixel groups per tile
     constexpr int kMB = PT / 32;                     // 32-pixel MFMA row blocks
-    static_assert((kNch & (kNch - 1)) == 0, "row swizzle needs a power-of-two chunk count");
-    __shared__ __align__(16) int8_t As[PT * C];
+    // A-tile rows of kNch 16-byte chunks: a power of two of them swizzled by the row, other counts
+    // padded by one chunk (16 consecutive rows then start on 16 distinct bank groups)
+    constexpr bool kPow2 = (kNch & (kNch - 1)) == 0;
+    constexpr int kPitch = kPow2 ? C : C + 16;
+    auto a_off = [](int p, int chunk) { return p * kPitch + ((kPow2 ? chunk ^ (p & (kNch - 1)) : chunk) << 4); };
+    __shared__ __align__(16) int8_t As[PT * kPitch];
     __shared__ float red[kNW][PT];
     __shared__ uint32_t redb[kNW][PT];
     __shared__ int nan_px[PT];
@@ -193,7 +200,7 @@ __global__ __launch_bounds__(128, convt_min_waves<KC>()) void convt_fused_kernel
         for (int k = 0; k < KC; k++) {
             const int c = cg + 32 * k;
             const uint32_t word = (e & 1) ? ((&v[k].x)[e >> 1] >> 16) : ((&v[k].x)[e >> 1] & 0xFFFFu);
-            As[p * C + ((((c >> 4) ^ (p & (kNch - 1)))) << 4) + (c & 15)] =
+            As[a_off(p, c >> 4) + (c & 15)] =
                 static_cast<int8_t>(qrow_bits(static_cast<uint16_t>(word), inv) & 0xFFu);
         }
     }
@@ -225,7 +232,7 @@ __global__ __launch_bounds__(128, convt_min_waves<KC>()) void convt_fused_kernel
 #pragma unroll
         for (int ks = 0; ks < KC; ks++) {
             const int c = 2 * ks + hi;
-            const v4i fa = *reinterpret_cast<const v4i*>(As + row * C + ((c ^ (row & (kNch - 1))) << 4));
+            const v4i fa = *reinterpret_cast<const v4i*>(As + a_off(row, c));
             acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[ks], fa, acc, 0, 0, 0);
         }
         if (row < np) {
@@ -300,9 +307,13 @@ extern "C" int forge_int8_conv_transpose2d_k2s2_forward(const uint16_t* input, c
         aligned(output, 4)) {
         const int hw = static_cast<int>(HW);
         switch (C_in) {
-            case 32:  return launch_convt_fused<1>(input, weight, w_scale, bias, output, N, hw, W, C_out, s);
-            case 64:  return launch_convt_fused<2>(input, weight, w_scale, bias, output, N, hw, W, C_out, s);
+            case 32: return launch_convt_fused<1>(input, weight, w_scale, bias, output, N, hw, W, C_out, s);
+            case 64: return launch_convt_fused<2>(input, weight, w_scale, bias, output, N, hw, W, C_out, s);
+            case 96: return launch_convt_fused<3>(input, weight, w_scale, bias, output, N, hw, W, C_out, s);
             case 128: return launch_convt_fused<4>(input, weight, w_scale, bias, output, N, hw, W, C_out, s);
+            case 160: return launch_convt_fused<5>(input, weight, w_scale, bias, output, N, hw, W, C_out, s);
+            case 192: return launch_convt_fused<6>(input, weight, w_scale, bias, output, N, hw, W, C_out, s);
+            case 224: return launch_convt_fused<7>(input, weight, w_scale, bias, output, N, hw, W, C_out, s);
             case 256: return launch_convt_fused<8>(input, weight, w_scale, bias, output, N, hw, W, C_out, s);
             default: break;
         }

@@ -270,3 +270,23 @@ def test_conv_transpose_special_pixels(dev, orc, C_in):
     out = buf[1:1 + want.size].view(want.shape)
     ops.int8_conv_transpose2d_k2s2_forward(xd, wd, wsd, bd, out=out)
     assert _bits_equal(to_host(out), want)
+
+
+@pytest.mark.parametrize("C_in", [96, 160, 192, 224])
+@pytest.mark.parametrize("N,H,W,C_out,bias", [(2, 13, 24, 9, True), (1, 5, 8, 40, False), (3, 1, 72, 1, True)])
+def test_conv_transpose_padded_rows(dev, orc, C_in, N, H, W, C_out, bias):
+    """The one-pass kernel at channel counts whose A-tile rows are padded: a last tile of 8 to 24
+    pixels, a NaN, an infinity and an all-zero pixel."""
+    from forge_amd import ops
+    rng = np.random.default_rng(C_in + H)
+    x = rng.uniform(-2, 2, (N, C_in, H, W)).astype(np.float16)
+    x[0, 3, 0, 1] = np.nan
+    x[0, 5, 0, 2] = np.inf
+    x[0, :, 0, 3] = 0
+    w = rng.integers(-127, 128, (4 * C_out, C_in)).astype(np.int8)
+    ws = rng.uniform(1e-3, 2e-2, C_out).astype(np.float16)
+    b = rng.uniform(-0.5, 0.5, C_out).astype(np.float16) if bias else None
+    say(f"conv_transpose padded rows C_in={C_in} N={N} H={H} W={W} C_out={C_out}")
+    y = to_host(ops.int8_conv_transpose2d_k2s2_forward(to_dev(x, dev), to_dev(w, dev), to_dev(ws, dev),
+                                                       None if b is None else to_dev(b, dev)))
+    assert _bits_equal(y, orc.conv_transpose2d_k2s2(x, w, ws, b))
