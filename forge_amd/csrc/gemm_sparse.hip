@@ -1020,13 +1020,18 @@ struct SpRingTile {
             for (int j = 0; j < kTM; j++) acc[i][j] = v4i{0, 0, 0, 0};
 
         const SpBufs bf = sp_bufs(W, X, meta, M, N, K);
+        // K % 128 = 64: the last stage is half past K. Tokens there read as zeros (offsets moved out of
+        // range), so what the other half of the weights and index words hold adds nothing; those too
+        // are moved out of range, which at the last row is the buffer's end.
         uint32_t ow[kWIns], ox[kXIns];
+        bool tw[kWIns], tx[kXIns];                          // chunk in the stage's second half
 #pragma unroll
         for (int q = 0; q < kWIns; q++) {
             const int s = (wave * kWIns + q) * kWave + lane;
             const int r = s >> 2, c = (s & 3) ^ lds_swz4(r);
             const int gr = (n0 + r) < N ? (n0 + r) : N - 1;
             ow[q] = static_cast<uint32_t>(gr) * Kc + 16 * c;
+            tw[q] = c >= 2;
         }
 #pragma unroll
         for (int q = 0; q < kXIns; q++) {
@@ -1034,24 +1039,28 @@ struct SpRingTile {
             const int r = s >> 3, c = (s & 7) ^ lds_swz8(r);
             const int gr = (m0 + r) < M ? (m0 + r) : M - 1;
             ox[q] = static_cast<uint32_t>(gr) * K + 16 * c;
+            tx[q] = c >= 4;
         }
         uint32_t oi;
+        bool ti;
         {
             const int s = wave * kILanes + (lane & (kILanes - 1));   // 16-byte chunk of the stage's index area
             int b = (n0 >> 4) + (s >> 4);
             b = b < (N >> 4) ? b : (N >> 4) - 1;
             oi = static_cast<uint32_t>(b) * cpr * 64 + 16 * (s & 15);
+            ti = (s & 15) >= 8;
         }
-        const int nst = K / 128;
+        const int nst = (K + 127) / 128;
         auto slot_of = [&](int st) { return lds + (st % D) * kSlotBytes; };
         auto issue = [&](int st) {
             int8_t* slot = slot_of(st);
             const uint32_t su = static_cast<uint32_t>(st);
+            const bool half = (st + 1) * 128 > K;
 #pragma unroll
-            for (int q = 0; q < kWIns; q++) dma16_buf(bf.w, ow[q], su * 64, slot + (wave * kWIns + q) * 1024);
+            for (int q = 0; q < kWIns; q++) dma16_buf(bf.w, half && tw[q] ? 0xC0000000u : ow[q], su * 64, slot + (wave * kWIns + q) * 1024);
 #pragma unroll
-            for (int q = 0; q < kXIns; q++) dma16_buf(bf.x, ox[q], su * 128, slot + kWBytes + (wave * kXIns + q) * 1024);
-            if (lane < kILanes) dma16_buf(bf.i, oi, su * 256, slot + kWBytes + kXBytes + wave * (16 * kILanes));
+            for (int q = 0; q < kXIns; q++) dma16_buf(bf.x, half && tx[q] ? 0xC0000000u : ox[q], su * 128, slot + kWBytes + (wave * kXIns + q) * 1024);
+            if (lane < kILanes) dma16_buf(bf.i, half && ti ? 0xC0000000u : oi, su * 256, slot + kWBytes + kXBytes + wave * (16 * kILanes));
         };
         // Waits for this wave's DMAs of stage kt when `later` stages were issued after it.
         auto wait_stage = [&](int later) {
@@ -1393,6 +1402,20 @@ int sparse_gemm(const int8_t* W_comp, const int8_t* x, const uint32_t* meta, con
                          : launch_sparse_dma<128, false, 128>(W_comp, x, meta, ep, K, s);
         return out16 ? launch_sparse_dma<128, true>(W_comp, x, meta, ep, K, s)
                      : launch_sparse_dma<128, false>(W_comp, x, meta, ep, K, s);
+    }
+    // K % 128 = 64: the ring engine, whose last stage is then half zeros, up to one round of its
+    // tiles or 24 stages; deep and large the register-staged 256 x 128 tiles read less. Linear
+    // layers, us, register-staged / ring: 1024 x 5184 x 1280 41.6 / 27.3, 150 x 2368 x 1664 20.7 /
+    // 12.9, 20000 x 2112 x 960 136 / 114, 43057 x 448 x 1728 235 / 158; beyond the line
+    // 2000 x 4160 x 4096 67 / 78, 8192 x 4160 x 8192 470 / 502.
+    const long long ring_tiles = static_cast<long long>(divup(N, kSpRingRows)) * divup(M, 64);
+    if (dma_fits && M > 64 && tile == FORGE_SPARSE_TILE_AUTO && static_cast<long long>(N) * K < (1LL << 31) &&
+        (steps <= 24 || ring_tiles <= static_cast<long long>(kSpRingPerCu) * cu_count_or_default())) {
+        void* o = out16 ? static_cast<void*>(out16) : static_cast<void*>(out32);
+        GemmEpilogue ep{out32, out16, act_scale, w_scale, bias, M, N, aligned(o, 16) ? 1 : 0};
+        note_route("ring64x64");
+        return out16 ? launch_sparse_ring<true, kSpRingRows, kSpRingDepth>(W_comp, x, meta, ep, K, s)
+                     : launch_sparse_ring<false, kSpRingRows, kSpRingDepth>(W_comp, x, meta, ep, K, s);
     }
     p.split_k = 1;
     p.steps_per_split = steps;

@@ -328,3 +328,35 @@ def test_sparse_256x256_int32_whole(dev, orc, M, K, N):
     assert ops.last_route() == "dma256x256"
     bad = int((got != ref).sum())
     assert bad == 0, f"{bad} of {got.size} outputs differ"
+
+
+# K % 128 = 64 on the ring engine: a last stage half past K, at one to several stages, ragged token and
+# weight tiles, the operands' last row at the end of its buffer; beyond 24 stages past one round of
+# tiles the register-staged engine.
+@pytest.mark.parametrize("M,K,N,route", [(65, 64, 16, "ring64x64"), (100, 192, 80, "ring64x64"), (130, 448, 208, "ring64x64"),
+                                         (700, 1088, 1728, "ring64x64"), (1024, 5184, 144, "ring64x64"),
+                                         (2000, 3264, 2048, "regstaged")])
+def test_sparse_half_stage(dev, orc, M, K, N, route):
+    import torch
+    from forge_amd import ops
+    rng = np.random.default_rng(M + K + N)
+    W = int8_uniform(rng, (N, K))
+    x = int8_uniform(rng, (M, K))
+    act = rng.uniform(0.001, 0.05, M).astype(np.float32)
+    ws = rng.uniform(0.001, 0.05, N).astype(np.float16)
+    b = rng.uniform(-0.5, 0.5, N).astype(np.float16)
+    cr, mr = orc.prune_compress_24(W)
+    ref = orc.sparse_gemm_s32(cr, x, mr, N, K, threads=orc.cpu_threads())
+    comp, raw, meta = _prep(dev, W)
+    say(f"sparse half stage M={M} K={K} N={N}")
+    xd = to_dev(x, dev)
+    C = torch.empty((M, N), dtype=torch.int32, device=dev)
+    poison(C, 0x7B)
+    assert np.array_equal(to_host(ops.sparse_int8_gemm_s32(comp, xd, meta, out=C)), ref)
+    for bias in (b, None):
+        Y = torch.empty((M, N), dtype=torch.float16, device=dev)
+        poison(Y, 0x7B)
+        ops.sparse_int8_gemm(comp, xd, meta, to_dev(act, dev), to_dev(ws, dev), None if bias is None else to_dev(bias, dev),
+                             split_k=0, out=Y)
+        assert ops.last_route().startswith(route)
+        assert np.array_equal(to_host(Y).view(np.uint16), orc.dequant_epilogue(ref, act, ws, bias).view(np.uint16))
