@@ -194,9 +194,9 @@ def _prep_sparse(ops, W):
 
 PROBE_KERNELS = {
     # probe: (kernel-name substrings, any of which marks a dispatch of the probe)
-    "c2_gemm": ("gemm_dma_kernel<256, 256, true, forge_amd::DmaRowMajor>",),
+    "c2_gemm": ("gemm_ring_kernel<forge_amd::RingTile<256, 256, 4, 2, 2>, true, false",),
     "c3_sparse": ("sparse_wide_s32_kernel", "sparse_dma32_tail_kernel<false,", "sparse_dma32_kernel<false,"),
-    "c3_dense": ("gemm_dma_coltail_kernel<false>", "gemm_dma_kernel<256, 256, false, forge_amd::DmaRowMajor>"),
+    "c3_dense": ("gemm_ring_tail_kernel<false>", "gemm_ring_kernel<forge_amd::RingTile<256, 256, 4, 2, 2>, false, false"),
     "c5_conv": ("conv_window_kernel<7, 2, false>",),
     "c4_dense_M16": ("decode_dense_kernel<true",),
     "c4_sparse_M16": ("decode_sparse_reg_kernel<true",),
@@ -326,9 +326,9 @@ COUNTER_SETS = [
            "TCP_TCC_READ_REQ_LATENCY_sum"),
 ]
 PROBE_TITLES = {
-    "c2_gemm": "configs[1] GEMM 4096^3, FP16 out (`gemm_dma_kernel<256,256,true>`)",
+    "c2_gemm": "configs[1] GEMM 4096^3, FP16 out (`gemm_ring_kernel` on 256x256 tiles)",
     "c3_sparse": "configs[2] 2:4 sparse 4096x11008x4096, INT32 out (`sparse_wide_s32_kernel`: 256 tokens x 320-352 weight rows per tile, 2 tiles per CU)",
-    "c3_dense": "configs[2] shape dense, INT32 out (`gemm_dma_coltail_kernel<false>`: 256- and 192-row tiles, one launch)",
+    "c3_dense": "configs[2] shape dense, INT32 out (`gemm_ring_tail_kernel<false>`: 256- and 192-row tiles, one launch)",
     "c5_conv": "configs[4] NHWC conv, INT32 out (`conv_window_kernel<7,2,false>`: 224-pixel x 256-channel tiles, input window in LDS once per channel chunk)",
     "c4_dense_M16": "configs[3] M=16 dense decode GEMM (`decode_dense_kernel`)",
     "c4_sparse_M16": "configs[3] M=16 2:4 decode GEMM (`decode_sparse_reg_kernel`)",
@@ -1060,7 +1060,7 @@ def main() -> int:
         "roofline": {"bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_INT8_TOPS,
                      "unit": "TOPS", "frac": round(achieved / PEAK_INT8_TOPS, 4), "traffic": measured_traffic(),
                      "mfma_busy": measured_mfma_busy(),
-                     "kernel": "gemm_dma_kernel<256,256,dequant>", "kernel_ms": round(t_gemm, 5),
+                     "kernel": "gemm_ring_kernel<RingTile<256,256,4,2,2>,dequant>", "kernel_ms": round(t_gemm, 5),
                      "quantize_ms": round(t_q, 5)},
     }
     if not args.no_cpu:

@@ -27,7 +27,7 @@ __global__ __launch_bounds__(256) void probe_mfma_lds_kernel(const int8_t* __res
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     const int wm = (wave >> 1) * 128, wn = (wave & 1) * 128;
     const int l31 = lane & 31, hi = lane >> 5;
-    // one stage: A rows (tile-local 0..255) then B rows, 128 bytes each, chunk swizzle of DmaTile
+    // one stage: A rows (tile-local 0..255) then B rows, 128 bytes each, chunk swizzle lds_swz8
     const int8_t* a = A + static_cast<size_t>(blockIdx.x % tiles_a) * 256 * 128;
     const int8_t* b = B + static_cast<size_t>(blockIdx.x % tiles_a) * 256 * 128;
     for (int s = threadIdx.x; s < 2 * 256 * 8; s += 256) {
