@@ -21,6 +21,7 @@ from typing import Optional
 
 import torch
 from torch import nn
+from torch.autograd import forward_ad
 
 from . import ops
 
@@ -37,6 +38,18 @@ def _as_weight(weight_fp: torch.Tensor, dev: torch.device) -> torch.Tensor:
     return w.to(dev).contiguous()
 
 
+def _plain(*tensors: torch.Tensor) -> bool:
+    """Whether a foreign call on the tensors' addresses can stand for torch operators on them: no
+    tensor without memory of its own (batched gradients, zero tensors, fake and other subclasses), no
+    dispatch mode that has to see the operators (tracing), no forward-mode tangents."""
+    if torch._C._len_torch_dispatch_stack() or forward_ad._current_level >= 0:
+        return False
+    for t in tensors:
+        if type(t) not in (torch.Tensor, nn.Parameter) or not torch._C._has_storage(t) or t._is_zerotensor():
+            return False
+    return True
+
+
 class _Int8LinearFn(torch.autograd.Function):
     """Forward on the INT8 path; backward through the dequantized FP16 weight, returning the
     input and bias gradients (the reference's _Int8LinearFn, linear.py:115-132)."""
@@ -51,10 +64,12 @@ class _Int8LinearFn(torch.autograd.Function):
     def backward(ctx, grad_output):
         w_int8, w_scale = ctx.saved_tensors
         g = grad_output if grad_output.dtype == torch.float16 else grad_output.to(torch.float16)
-        # With gradients recorded (create_graph=True) the torch operators below carry them; the
-        # library's passes would not. It sums whole FP16 vectors of a non-empty batch.
-        if (not torch.is_grad_enabled() and grad_output.dtype == torch.float16 and g.is_cuda and w_int8.is_cuda
-                and w_int8.is_contiguous() and w_scale.dtype == torch.float16 and g.shape[0] > 0 and g.shape[1] >= 8):
+        # With gradients recorded (create_graph=True), batched or traced the torch operators below
+        # carry them; the library's passes would not. Saved-tensor hooks may have changed layouts and
+        # devices. The library sums whole FP16 vectors of a non-empty batch.
+        if (not torch.is_grad_enabled() and grad_output.dtype == torch.float16 and _plain(g, w_int8, w_scale)
+                and g.is_cuda and w_int8.device == g.device and w_scale.device == g.device and w_int8.is_contiguous()
+                and w_scale.is_contiguous() and w_scale.dtype == torch.float16 and g.shape[0] > 0 and g.shape[1] >= 8):
             if not g.is_contiguous():
                 g = g.contiguous()
             w16, grad_bias = ops.int8_linear_backward_prep(w_int8, w_scale, g, ctx.has_bias)

@@ -98,6 +98,43 @@ def test_linear_backward_passes(dev, M, K, N):
     assert float((gb.float() - gb2.float()).abs().max()) <= float(g.float().abs().sum(0).max()) * (M * 2.0 ** -24 + 2.0 ** -10)
 
 
+def test_linear_backward_transformed(dev):
+    """Gradients that are batched, traced, dual or behind saved-tensor hooks equal those through the
+    torch operators: the passes on raw addresses stand aside. Gradients of one token and small
+    integers, so every sum is exact and the values are compared exactly."""
+    import torch
+    import torch.autograd.forward_ad as fwAD
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from forge_amd.nn import QuantizedLinear
+    K, N = 32, 16
+    rng = np.random.default_rng(5)
+    m = QuantizedLinear(K, N).to(dev)
+    m.w_int8.copy_(to_dev(rng.integers(-8, 9, (N, K)).astype(np.int8), dev))
+    m.w_scale.data.copy_(to_dev(rng.choice([0.5, 0.25, 1.0], N).astype(np.float16), dev))
+    x = to_dev(fp16_normal(rng, (1, K)), dev).requires_grad_(True)
+    w = (m.w_int8.half() * m.w_scale.detach()[:, None])
+    g = torch.from_numpy(rng.integers(-3, 4, (3, 1, N)).astype(np.float16)).to(dev)
+    say("linear backward transformed")
+    y = m(x)
+    gx, gb = torch.autograd.grad(y, (x, m.bias), g, is_grads_batched=True, retain_graph=True)
+    assert torch.equal(gx, (g.float() @ w.float()).half()) and torch.equal(gb, g[:, 0])
+    jac = torch.autograd.functional.jacobian(m, x.detach(), vectorize=True)
+    assert torch.equal(jac[0, :, 0], w)
+    with fwAD.dual_level():
+        r = torch.autograd.grad(y, (x, m.bias), fwAD.make_dual(g[0], g[1]), retain_graph=True)
+        tx, tb = (fwAD.unpack_dual(t).tangent for t in r)
+    assert torch.equal(tx, (g[1].float() @ w.float()).half()) and torch.equal(tb, g[1, 0])
+    traced = make_fx(lambda t: torch.autograd.grad(y, (x, m.bias), t, retain_graph=True))(g[0])
+    for t in (g[0], g[1]):
+        gx, gb = traced(t)
+        assert torch.equal(gx, (t.float() @ w.float()).half()) and torch.equal(gb, t[0])
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.t().contiguous().t() if t.dim() == 2 else
+                                                  torch.stack([t, t], 1)[:, 0]):
+        y = m(x)
+    gx, gb = torch.autograd.grad(y, (x, m.bias), g[2])
+    assert torch.equal(gx, (g[2].float() @ w.float()).half()) and torch.equal(gb, g[2, 0])
+
+
 @pytest.mark.parametrize("M,K,N,bias", [(5, 256, 64, True), (200, 1280, 320, True), (129, 512, 96, False)])
 def test_sparse_linear(dev, orc, M, K, N, bias):
     import torch

@@ -73,3 +73,41 @@ def test_reference_state_dict_bad_w_meta_shape(orc):
     sd["w_meta"] = sd["w_meta"][:, :2]
     with pytest.raises(RuntimeError, match="w_meta"):
         SparseLinear(128, 32).load_state_dict(sd)
+
+
+def test_plain_tensors():
+    """What may go to the library by address in a backward: plain tensors with memory of their own, and
+    nothing while a transform has to see the operators."""
+    import torch.autograd.forward_ad as fwAD
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.utils.flop_counter import FlopCounterMode
+    from forge_amd.nn import _plain
+    t = torch.ones(3, 4)
+    assert _plain(t, torch.nn.Parameter(t), t.t())
+    assert not _plain(t, torch._efficientzerotensor(3))
+    seen = []
+    torch.vmap(lambda a: (seen.append(_plain(t, a)), a)[1])(t)
+    x = torch.ones(4, requires_grad=True)
+
+    class Probe(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, a):
+            return a * 1
+
+        @staticmethod
+        def backward(ctx, g):
+            seen.append(_plain(g))
+            return g
+
+    torch.autograd.grad(Probe.apply(x), x, t, is_grads_batched=True)
+    assert seen == [False, False]
+    torch.autograd.grad(Probe.apply(x), x, t[0])
+    assert seen.pop()
+    with FakeTensorMode():
+        fake = torch.ones(3)
+    assert not _plain(fake)
+    with fwAD.dual_level():
+        assert not _plain(t)
+    with FlopCounterMode(display=False):
+        assert not _plain(t)
+    assert _plain(t)
