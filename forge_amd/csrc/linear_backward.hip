@@ -136,22 +136,27 @@ extern "C" int forge_int8_linear_backward_prep(const int8_t* w, const uint16_t* 
                                                const uint16_t* grad, float* partial, uint16_t* grad_bias, int M, int K,
                                                int N, void* stream)
 {
-    if (M <= 0 || N <= 0 || K <= 0) return FORGE_OK;
-    if (!w || !w_scale || !w16t || (grad_bias && (!grad || !partial || N < 8))) return FORGE_EINVAL;
+    // No columns of the weight (K = 0): nothing to convert. No rows of the gradient (M = 0): its sums are 0.
+    if (M < 0 || N <= 0 || K < 0) return FORGE_OK;
+    if (!w_scale || (K > 0 && (!w || !w16t)) || (grad_bias && (!partial || N < 8 || (M > 0 && !grad)))) return FORGE_EINVAL;
     hipStream_t s = as_stream(stream);
-    const int by = divup(N, 64);
-    if (by > 65535) return FORGE_EINVAL;
-    const dim3 grid(static_cast<unsigned>(divup(K, 64)), static_cast<unsigned>(by));
-    if (K % 16 == 0 && aligned(w, 16))
-        dequantize_weight_t_kernel<true><<<grid, 256, 0, s>>>(w, w_scale, w16t, N, K);
-    else
-        dequantize_weight_t_kernel<false><<<grid, 256, 0, s>>>(w, w_scale, w16t, N, K);
-    int st = launch_status();
-    if (st != FORGE_OK || !grad_bias) return st;
+    int st = FORGE_OK;
+    if (K > 0) {
+        const int by = divup(N, 64);
+        if (by > 65535) return FORGE_EINVAL;
+        const dim3 grid(static_cast<unsigned>(divup(K, 64)), static_cast<unsigned>(by));
+        if (K % 16 == 0 && aligned(w, 16))
+            dequantize_weight_t_kernel<true><<<grid, 256, 0, s>>>(w, w_scale, w16t, N, K);
+        else
+            dequantize_weight_t_kernel<false><<<grid, 256, 0, s>>>(w, w_scale, w16t, N, K);
+        if ((st = launch_status()) != FORGE_OK) return st;
+    }
+    if (!grad_bias) return FORGE_OK;
     // 16 rows a pass of a workgroup's four waves; FORGE_COLUMN_SUM_PARTS parts at most
     const int rows = std::max(16, divup(divup(M, FORGE_COLUMN_SUM_PARTS), 16) * 16), parts = divup(M, rows);
-    column_sum_kernel<<<dim3(static_cast<unsigned>(divup(N, 512)), static_cast<unsigned>(parts)), 256, 0, s>>>(grad, partial,
-                                                                                                               M, N, rows);
+    if (parts > 0)
+        column_sum_kernel<<<dim3(static_cast<unsigned>(divup(N, 512)), static_cast<unsigned>(parts)), 256, 0, s>>>(
+            grad, partial, M, N, rows);
     if ((st = launch_status()) != FORGE_OK) return st;
     column_sum_finish_kernel<<<static_cast<unsigned>(divup(N, 256)), 256, 0, s>>>(partial, grad_bias, N, parts);
     return launch_status();

@@ -162,8 +162,8 @@ int forge_int8_gemm_s32(const int8_t* A, const int8_t* B, int32_t* C,
  * python/forge/nn/linear.py:115-132): the passes around the matrix product of int8_linear's
  * backward. w16t (K, N) fp16: w16t[k,n] = half((float)w[n,k] * w_scale[n]), so that the input
  * gradient is grad (M, N) times its transpose. With grad_bias (N) fp16 non-null (N >= 8): the column
- * sums of grad, accumulated in fp32 in a fixed order; partial: scratch of FORGE_COLUMN_SUM_PARTS * N
- * floats. */
+ * sums of grad, accumulated in fp32 in a fixed order (zeros at M = 0); partial: scratch of
+ * FORGE_COLUMN_SUM_PARTS * N floats. */
 #define FORGE_COLUMN_SUM_PARTS 32
 int forge_int8_linear_backward_prep(const int8_t* w, const uint16_t* w_scale, uint16_t* w16t, const uint16_t* grad,
                                     float* partial, uint16_t* grad_bias, int M, int K, int N, void* stream);

@@ -98,6 +98,35 @@ def test_linear_backward_passes(dev, M, K, N):
     assert float((gb.float() - gb2.float()).abs().max()) <= float(g.float().abs().sum(0).max()) * (M * 2.0 ** -24 + 2.0 ** -10)
 
 
+def test_linear_backward_empty(dev):
+    """No columns of the weight: the bias gradient is still the column sum. No tokens: it is zero. Buffers
+    of both sizes are filled and freed first, so that fresh memory is not zero by chance."""
+    import torch
+    from forge_amd import ops
+    from forge_amd.nn import QuantizedLinear
+    N = 24
+    g = torch.arange(5 * N, device=dev).reshape(5, N).half()
+    ws = torch.ones(N, dtype=torch.float16, device=dev)
+    say("linear backward empty")
+
+    def stale():
+        del_me = [torch.full((n,), 7.0, dtype=torch.float16, device=dev) for n in (N, 64 * N)]
+        del del_me
+
+    stale()
+    w16, gb = ops.int8_linear_backward_prep(torch.empty((N, 0), dtype=torch.int8, device=dev), ws, g, True)
+    assert w16.shape == (N, 0) and torch.equal(gb, g.sum(0))
+    stale()
+    w = torch.ones((N, 32), dtype=torch.int8, device=dev)
+    w16, gb = ops.int8_linear_backward_prep(w, ws, g[:0], True)
+    assert torch.equal(w16, w.half()) and torch.equal(gb, torch.zeros_like(gb))
+    stale()
+    m = QuantizedLinear(0, N).to(dev)
+    x = torch.empty((5, 0), dtype=torch.float16, device=dev, requires_grad=True)
+    gx, gb = torch.autograd.grad(m(x), (x, m.bias), g)
+    assert gx.shape == (5, 0) and torch.equal(gb, g.sum(0))
+
+
 def test_linear_backward_transformed(dev):
     """Gradients that are batched, traced, dual or behind saved-tensor hooks equal those through the
     torch operators: the passes on raw addresses stand aside. Gradients of one token and small
