@@ -4,6 +4,7 @@
 #include "forge_amd.h"
 
 #include <algorithm>
+#include <climits>
 
 namespace forge_amd {
 
@@ -15,12 +16,16 @@ namespace forge_amd {
 template <bool VEC>
 __global__ __launch_bounds__(256) void dequantize_weight_t_kernel(const int8_t* __restrict__ w,
                                                                   const uint16_t* __restrict__ w_scale,
-                                                                  uint16_t* __restrict__ out, int N, int K)
+                                                                  uint16_t* __restrict__ out, int N, int K,
+                                                                  unsigned tiles_k, unsigned tiles)
 {
     constexpr int kT = 64, kPitch = kT + 4;
     __shared__ __align__(16) int8_t tile[kT * kPitch];
     const int t = threadIdx.x;
-    const int n0 = blockIdx.y * kT, k0 = blockIdx.x * kT;
+    // 64 x 64 tiles numbered along K first over both grid dimensions, which alone end at 65535 rows of tiles
+    const unsigned id = blockIdx.y * gridDim.x + blockIdx.x;
+    if (id >= tiles) return;
+    const int n0 = static_cast<int>(id / tiles_k) * kT, k0 = static_cast<int>(id % tiles_k) * kT;
     {
         const int r = t >> 2, c = 16 * (t & 3);        // 16 bytes of row n0 + r
         const int n = n0 + r, k = k0 + c;
@@ -142,13 +147,15 @@ extern "C" int forge_int8_linear_backward_prep(const int8_t* w, const uint16_t* 
     hipStream_t s = as_stream(stream);
     int st = FORGE_OK;
     if (K > 0) {
-        const int by = divup(N, 64);
-        if (by > 65535) return FORGE_EINVAL;
-        const dim3 grid(static_cast<unsigned>(divup(K, 64)), static_cast<unsigned>(by));
+        const long long tiles_k = divup(K, 64), tiles = tiles_k * divup(N, 64);
+        if (tiles > INT_MAX) return FORGE_EINVAL;
+        const unsigned gx = static_cast<unsigned>(std::min<long long>(tiles, 1 << 16));
+        const dim3 grid(gx, static_cast<unsigned>(divupll(tiles, gx)));
+        const unsigned tk = static_cast<unsigned>(tiles_k), nt = static_cast<unsigned>(tiles);
         if (K % 16 == 0 && aligned(w, 16))
-            dequantize_weight_t_kernel<true><<<grid, 256, 0, s>>>(w, w_scale, w16t, N, K);
+            dequantize_weight_t_kernel<true><<<grid, 256, 0, s>>>(w, w_scale, w16t, N, K, tk, nt);
         else
-            dequantize_weight_t_kernel<false><<<grid, 256, 0, s>>>(w, w_scale, w16t, N, K);
+            dequantize_weight_t_kernel<false><<<grid, 256, 0, s>>>(w, w_scale, w16t, N, K, tk, nt);
         if ((st = launch_status()) != FORGE_OK) return st;
     }
     if (!grad_bias) return FORGE_OK;

@@ -98,6 +98,20 @@ def test_linear_backward_passes(dev, M, K, N):
     assert float((gb.float() - gb2.float()).abs().max()) <= float(g.float().abs().sum(0).max()) * (M * 2.0 ** -24 + 2.0 ** -10)
 
 
+@pytest.mark.parametrize("N,K", [(65535 * 64 + 70, 3), (65536 * 64 + 64, 16), (9, 65536 * 64 + 17)])
+def test_linear_backward_many_tiles(dev, N, K):
+    """More than 65535 rows or columns of 64 x 64 weight tiles, and more tiles than one grid dimension."""
+    import torch
+    from forge_amd import ops
+    gen = torch.Generator(device=dev).manual_seed(N)
+    w = torch.randint(-127, 128, (N, K), dtype=torch.int8, device=dev, generator=gen)
+    ws = (torch.rand(N, device=dev, generator=gen) * 0.01 + 0.001).half()
+    g = torch.ones((1, N), dtype=torch.float16, device=dev)
+    say(f"linear backward many tiles N={N} K={K}")
+    w16, gb = ops.int8_linear_backward_prep(w, ws, g, True)
+    assert torch.equal(w16, w.half() * ws[:, None]) and torch.equal(gb, g[0])
+
+
 def test_linear_backward_empty(dev):
     """No columns of the weight: the bias gradient is still the column sum. No tokens: it is zero. Buffers
     of both sizes are filled and freed first, so that fresh memory is not zero by chance."""
