@@ -218,6 +218,8 @@ def int8_linear_backward_prep(w_int8: torch.Tensor, w_scale: torch.Tensor, grad:
     """What int8_linear's input gradient multiplies grad (M, N) with, the FP16 weight as an (N, K)
     tensor contiguous along N, and the bias gradient (N,) or None (N >= 8)."""
     N, K = w_int8.shape
+    if grad.dim() != 2 or grad.shape[1] != N:
+        raise ValueError(f"grad must be (M, {N}), got {tuple(grad.shape)}")
     _need(w_int8, torch.int8, "w_int8")
     _need(w_scale, torch.float16, "w_scale", N)
     _need(grad, torch.float16, "grad")

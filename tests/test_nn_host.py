@@ -111,3 +111,12 @@ def test_plain_tensors():
     with FlopCounterMode(display=False):
         assert not _plain(t)
     assert _plain(t)
+
+
+@pytest.mark.parametrize("shape", [(5, 15), (5, 17), (80,), (5, 16, 1), (16, 5)])
+def test_backward_prep_refuses_other_shapes(shape):
+    """A gradient that is not (M, N) is refused before anything is launched on it."""
+    from forge_amd import ops
+    w, ws = torch.zeros((16, 32), dtype=torch.int8), torch.ones(16, dtype=torch.float16)
+    with pytest.raises(ValueError, match="grad must be"):
+        ops.int8_linear_backward_prep(w, ws, torch.zeros(shape, dtype=torch.float16), True)
