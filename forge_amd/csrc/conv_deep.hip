@@ -492,7 +492,11 @@ int launch_conv_deep(const ConvDeepShape& c, void* workspace, size_t ws_bytes, h
     a.tiles_w = divup(c.Wo, a.Wt);
     const long long tiles = static_cast<long long>(a.tiles_h) * a.tiles_w;
 
-    // workspace: fragments, then the channel maxima of as many images as fit
+    // workspace: fragments (16-byte vectors and LDS DMA, so from its first 16-byte boundary on: the caller's
+    // buffer may start anywhere), then the channel maxima of as many images as fit
+    const size_t skip = -reinterpret_cast<uintptr_t>(workspace) & 15;
+    if (ws_bytes < skip) return -1;
+    ws_bytes -= skip;
     const long long nfrag = static_cast<long long>(groups_co) * ncb * a.nc * taps * 64;
     const long long wbytes = 16 * nfrag;
     const long long HW = static_cast<long long>(c.H) * c.W;
@@ -507,7 +511,7 @@ int launch_conv_deep(const ConvDeepShape& c, void* workspace, size_t ws_bytes, h
     a.mg_g = udiv_multiplier(a.G);
     a.mg_tiles = udiv_multiplier(a.tiles);
     a.mg_tw = udiv_multiplier(a.tiles_w);
-    int8_t* wf = static_cast<int8_t*>(workspace);
+    int8_t* wf = static_cast<int8_t*>(workspace) + skip;
     uint16_t* amax = reinterpret_cast<uint16_t*>(wf + wbytes);
     a.wf = wf;
     a.amax = amax;

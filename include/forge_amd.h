@@ -253,7 +253,8 @@ size_t forge_int8_conv2d_workspace_size(int C_in, int H, int W, int C_out, int k
 
 /* Replaces forge::nn::int8_conv2d_forward (include/forge/nn/int8_conv2d.cuh:41-53):
  * NCHW fp16 input, weight (C_out, C_in*kH*kW) int8, per-patch-row activation
- * quantization, dequant + bias, NCHW fp16 output. */
+ * quantization, dequant + bias, NCHW fp16 output. workspace: the bytes of the size above, at any
+ * alignment; its contents are scratch, and calls on several streams need one each. */
 int forge_int8_conv2d_forward(const uint16_t* input, const int8_t* weight,
                               const uint16_t* w_scale, const uint16_t* bias, uint16_t* output,
                               int N, int C_in, int H, int W, int C_out, int kH, int kW,

@@ -349,3 +349,25 @@ def test_conv_nchw_deep_special_values(dev, orc, W):
     y1 = to_host(ops.int8_conv2d_forward(buf[1:].view(N, C, H, W), to_dev(w, dev), to_dev(ws, dev), to_dev(b, dev), 3, 3,
                                          (1, 1)))
     assert np.array_equal(y1.view(np.uint16), y.view(np.uint16))
+
+
+@pytest.mark.parametrize("offset", [1, 2, 8, 15])
+def test_conv_nchw_deep_workspace_alignment(dev, orc, offset):
+    """The workspace may start at any byte: nothing outside it is written, and the bits are the same."""
+    import torch
+    from forge_amd import ops
+    rng = np.random.default_rng(offset)
+    N, C, H, W, Co = 3, 80, 41, 35, 72
+    x = rng.uniform(-1, 1, (N, C, H, W)).astype(np.float16)
+    w = int8_uniform(rng, (Co, C * 9))
+    ws = rng.uniform(0.005, 0.05, Co).astype(np.float16)
+    n = ops.int8_conv2d_workspace_size(C, H, W, Co, 3, 3, 1, 1, 1, 1)
+    buf = torch.full((n + 32,), 0x5A, dtype=torch.uint8, device=dev)
+    assert buf.data_ptr() % 16 == 0
+    say(f"conv nchw deep workspace offset={offset}")
+    y = to_host(ops.int8_conv2d_forward(to_dev(x, dev), to_dev(w, dev), to_dev(ws, dev), None, 3, 3, (1, 1),
+                                        workspace=buf[offset:offset + n]))
+    assert ops.last_route().startswith("conv-nchw-deep")
+    _nchw_check(orc, y, x, w, ws, None, 3, 1, 1, 1)
+    got = to_host(buf)
+    assert (got[:offset] == 0x5A).all() and (got[offset + n:] == 0x5A).all()
