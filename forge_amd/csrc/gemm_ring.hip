@@ -273,9 +273,10 @@ int launch_ring_conv(const ConvGeom& g, const int8_t* w, const GemmEpilogue& ep,
 {
     const int K = g.K;
     const long long img = static_cast<long long>(g.rows / (g.Ho * g.Wo)) * g.H * g.W * g.C;
-    // one buffer resource per operand, and udiv_magic's range for the chunk and pixel divisions
+    // one buffer resource per operand, and udiv_magic's range for the chunk, tap and pixel divisions
+    const long long k_end = static_cast<long long>(K) + 8 * kBK;
     if (img >= (1LL << 31) || static_cast<long long>(ep.N) * K >= (1LL << 31) || K > (1 << 30) ||
-        (static_cast<long long>(K) + 8 * kBK) * g.C >= (1LL << 32) ||
+        k_end * g.C >= (1LL << 32) || (k_end / g.C + 1) * g.kW >= (1LL << 32) ||
         static_cast<long long>(g.rows) * (g.Ho > g.Wo ? g.Ho : g.Wo) >= (1LL << 32))
         return -1;
     RingConv a;

@@ -67,7 +67,7 @@ struct RingRowMajor {
 // Implicit im2col of an NHWC image with C % 16 == 0 (K order (kh, kw, c)): a 16-byte chunk is 16
 // channels of one tap, so each lane finds its chunk's tap by two magic divisions per stage; a tap
 // in the padding gets an offset past the image, which reads as zeros. Needs an image under 2^31
-// bytes, (K + 8 stages) C < 2^32 and rows max(Ho, Wo) < 2^32.
+// bytes, (K + 8 stages) C < 2^32, ((K + 8 stages) / C + 1) kW < 2^32 and rows max(Ho, Wo) < 2^32.
 struct RingConv : ConvGeom {
     uint32_t x_bytes;
     uint32_t mg_c, mg_kw, mg_wo, mg_ho;   // udiv_magic multipliers of C, kW, Wo, Ho

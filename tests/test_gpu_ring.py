@@ -74,6 +74,20 @@ def test_ring_conv(dev, orc, N, H, W, C, Co, k, pad, stride, dil):
                           orc.dequant_epilogue(acc, act, ws, b).view(np.uint16))
 
 
+def test_conv_very_wide_kernel(dev, orc):
+    """A kernel of 65537 columns: past the range in which the gather's division of the tap by kW is
+    exact, so the register-staged gather, which divides truly, runs."""
+    from forge_amd import ops
+    rng = np.random.default_rng(9)
+    x, w = int8_uniform(rng, (1, 3, 65541, 16)), int8_uniform(rng, (24, 1, 65537, 16))
+    say("conv of 65537 columns")
+    got = to_host(ops.int8_conv2d_nhwc_s32(to_dev(x, dev), to_dev(w, dev)))
+    assert ops.last_route().startswith("regstaged")
+    for j in range(5):
+        want = x[0, :, j:j + 65537].reshape(3, -1).astype(np.int64) @ w.reshape(24, -1).T.astype(np.int64)
+        assert np.array_equal(got[0, :, j], want)
+
+
 @pytest.mark.parametrize("N,C_in,H,W,C_out,bias,route", [
     (1, 48, 7, 12, 5, True, "dma64x64 scatter"), (2, 80, 9, 13, 17, False, "dma64x64 scatter"),   # W % 4 = 0 and not
     (3, 16, 120, 132, 160, True, "dma128x128 scatter"), (2, 272, 100, 120, 96, True, "dma256x256 scatter"),
