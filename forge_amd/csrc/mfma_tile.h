@@ -110,7 +110,7 @@ __device__ __forceinline__ void lds_barrier() {
 
 // Row-major (rows, K) int8 matrix; needs K % 16 == 0 and a 16-byte aligned base.
 struct RowMajorOperand {
-    static constexpr bool kFix = false;
+    static constexpr bool kFix = false, kBytes = false;   // chunks shifted at the row's end; read byte by byte
     const int8_t* p;
     int rows;
     int K;
@@ -137,7 +137,7 @@ struct RowMajorOperand {
 // loads per chunk, 11.2 with the shift between the loads, 8.2 with it after them; 8192 x 1001 x 4096
 // with its quantizer 467 -> 109 us.
 struct RowMajorBytes {
-    static constexpr bool kFix = true;
+    static constexpr bool kFix = true, kBytes = false;
     const int8_t* p;
     int rows;
     int K;
@@ -173,7 +173,7 @@ struct RowMajorBytes {
 
 // Rows under 16 bytes: byte gathers.
 struct RowMajorShort {
-    static constexpr bool kFix = false;
+    static constexpr bool kFix = false, kBytes = true;
     const int8_t* p;
     int rows;
     int K;
@@ -207,7 +207,7 @@ struct ConvGeom {
 
 // Needs C % 16 == 0 (a chunk never straddles two taps) and a 16-byte aligned image.
 struct ConvOperand : ConvGeom {
-    static constexpr bool kFix = false;
+    static constexpr bool kFix = false, kBytes = false;
     struct Row { const int8_t* img; int hb, wb; };
     __device__ __forceinline__ Row row(int r) const {
         r = r < rows ? r : rows - 1;
@@ -231,7 +231,7 @@ struct ConvOperand : ConvGeom {
 
 // Same geometry, any C and alignment (byte gathers; odd shapes only).
 struct ConvBytes : ConvGeom {
-    static constexpr bool kFix = false;
+    static constexpr bool kFix = false, kBytes = true;
     struct Row { const int8_t* img; int hb, wb; };
     __device__ __forceinline__ Row row(int r) const {
         r = r < rows ? r : rows - 1;
@@ -312,10 +312,12 @@ struct NtTile {
 #pragma unroll
         for (int i = 0; i < kBPass; i++) rb[i] = opb.row(n0 + rr + kRowsPerPass * i);
 
-        // kS stages of loads in flight in registers (one on 256 x 256 tiles, whose accumulators leave
-        // room for no more): the loop is unrolled by kS, so that each stage's set is known at compile
-        // time.
-        constexpr int kS = BM * BN >= 256 * 256 ? 1 : 3;
+        // kS stages of loads in flight in registers: the loop is unrolled by kS, so that each stage's
+        // set is known at compile time. One on 256 x 256 tiles, whose accumulators leave room for no
+        // more, and where an operand is gathered byte by byte: its 16 loads and masks per chunk, three
+        // times over, cost more than they hide (NHWC 3x3, us, one stage in flight / three: 4 channels to
+        // 1024 on eight 52 x 73 images 64 / 115, 3 to 320 on four 40 x 82 19.4 / 31.6; on 64 x 64 tiles level).
+        constexpr int kS = BM * BN >= 256 * 256 || OpA::kBytes || OpB::kBytes ? 1 : 3;
         int4 sa[kS][kAPass], sb[kS][kBPass];
         auto gload = [&](int kt, int set) {
             const int k = kt * kBK + 16 * cc;
