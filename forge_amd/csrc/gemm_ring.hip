@@ -78,8 +78,8 @@ int ring_pick(int M, int N, int K, int cu, unsigned allowed, float* cost) {
 
 // ---- kernels ------------------------------------------------------------------------------
 
-template <class T, bool DEQUANT, bool UP, class OpA>
-__device__ __forceinline__ void ring_tile_at(const OpA& opa, const RingRowMajor& opb, const GemmEpilogue& ep,
+template <class T, bool DEQUANT, bool UP, class OpA, class OpB>
+__device__ __forceinline__ void ring_tile_at(const OpA& opa, const OpB& opb, const GemmEpilogue& ep,
                                              int K, int m0, int n0, int8_t* lds)
 {
     T t;
@@ -104,8 +104,8 @@ __device__ __forceinline__ void ring_coords(int bid, int tiles_m, int tiles_n, i
     tn = tn < tiles_n ? tn : tn - tiles_n;
 }
 
-template <class T, bool DEQUANT, bool UP, class OpA>
-__global__ __launch_bounds__(T::kThreads) void gemm_ring_kernel(OpA opa, RingRowMajor opb, GemmEpilogue ep,
+template <class T, bool DEQUANT, bool UP, class OpA, class OpB>
+__global__ __launch_bounds__(T::kThreads) void gemm_ring_kernel(OpA opa, OpB opb, GemmEpilogue ep,
                                                                 int tiles_m, int tiles_n, int K)
 {
     extern __shared__ __align__(16) int8_t lds[];
@@ -143,8 +143,8 @@ static int ring_allow_lds(Kern kern, int lds) {
     return e == hipSuccess ? FORGE_OK : static_cast<int>(e);
 }
 
-template <class T, bool DEQUANT, bool UP, class OpA>
-static int launch_ring_tile(const OpA& opa, const RingRowMajor& opb, const GemmEpilogue& ep, int K,
+template <class T, bool DEQUANT, bool UP, class OpA, class OpB>
+static int launch_ring_tile(const OpA& opa, const OpB& opb, const GemmEpilogue& ep, int K,
                             hipStream_t s)
 {
     constexpr int lds = ring_lds_bytes<T, DEQUANT>();
@@ -152,7 +152,7 @@ static int launch_ring_tile(const OpA& opa, const RingRowMajor& opb, const GemmE
     const int tiles_m = divup(ep.M, T::kBM), tiles_n = divup(ep.N, T::kBN);
     const long long total = static_cast<long long>(tiles_m) * tiles_n;
     if (total > 0x7FFFFFFFLL) return FORGE_EINVAL;
-    auto kern = gemm_ring_kernel<T, DEQUANT, UP, OpA>;
+    auto kern = gemm_ring_kernel<T, DEQUANT, UP, OpA, OpB>;
     static const int attr = ring_allow_lds(kern, lds);
     if (attr != FORGE_OK) return attr;
     kern<<<static_cast<unsigned>(total), T::kThreads, lds, s>>>(opa, opb, ep, tiles_m, tiles_n, K);
@@ -199,8 +199,8 @@ static void note_shape(int shape)
 }
 
 // Every shape but 256 x 256.
-template <bool DEQUANT, class OpA>
-static int launch_ring_shape(int shape, const OpA& opa, const RingRowMajor& opb, const GemmEpilogue& ep, int K,
+template <bool DEQUANT, class OpA, class OpB>
+static int launch_ring_shape(int shape, const OpA& opa, const OpB& opb, const GemmEpilogue& ep, int K,
                              hipStream_t s)
 {
     switch (shape) {
@@ -289,12 +289,36 @@ int launch_ring_conv(const ConvGeom& g, const int8_t* w, const GemmEpilogue& ep,
     int st = FORGE_OK;
     const int cu = device_info(&st).cu_count;
     if (st != FORGE_OK) return st;
-    // The gather's lane state does not fit beside the 256 x 256 tile's registers (172 bytes of
-    // spills per lane), so conv calls go without that shape.
+    const RingRowMajor opb{w, ep.N, K};
+    const int kH = K / (g.C * g.kW);
+    const long long lead = (static_cast<long long>(g.padH) * g.W + g.padW) * g.C;
+    if (g.C % kBK == 0 && kH <= 16 && g.kW <= 16 && img + 2 * lead < (1LL << 31)) {
+        RingConvTap b;
+        static_cast<ConvGeom&>(b) = g;
+        b.lead = static_cast<uint32_t>(lead);
+        b.range = static_cast<uint32_t>(img + 2 * lead);
+        b.kH = kH;
+        b.cps = g.C / kBK;
+        b.mg_cps = udiv_multiplier(b.cps);
+        b.mg_kw = a.mg_kw;
+        b.mg_wo = a.mg_wo;
+        b.mg_ho = a.mg_ho;
+        // 256 x 256 from 8 stages on: with fewer, its epilogue, which nothing overlaps, is most of a tile
+        // (INT32 outputs, us, 256 x 256 / the next pick: 256 -> 512 1x1 on 25 maps of 36 x 59 29 / 23).
+        float cost = 0.0f;
+        const int shape = ring_pick(ep.M, ep.N, K, cu, (1u << (K >= 8 * kBK ? kRingShapes : k256x256)) - 1, &cost);
+        note_shape(shape);
+        const RingRowMajorEven even{opb};
+        if (shape == k256x256)
+            return ep.c16 ? launch_ring_tile<T256x256, true, false>(b, even, ep, K, s)
+                          : launch_ring_tile<T256x256, false, false>(b, even, ep, K, s);
+        return ep.c16 ? launch_ring_shape<true>(shape, b, even, ep, K, s) : launch_ring_shape<false>(shape, b, even, ep, K, s);
+    }
+    // This gather's lane state does not fit beside the 256 x 256 tile's registers (172 bytes of
+    // spills per lane), so these calls go without that shape.
     float cost = 0.0f;
     const int shape = ring_pick(ep.M, ep.N, K, cu, (1u << k256x256) - 1, &cost);
     note_shape(shape);
-    const RingRowMajor opb{w, ep.N, K};
     return ep.c16 ? launch_ring_shape<true>(shape, a, opb, ep, K, s) : launch_ring_shape<false>(shape, a, opb, ep, K, s);
 }
 

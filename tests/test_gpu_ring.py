@@ -53,6 +53,10 @@ def test_ring_shapes(dev, orc, M, K, N, route):
     (2, 24, 24, 320, 192, 1, 0, 1, 1),     # pointwise
 ])
 def test_ring_conv(dev, orc, N, H, W, C, Co, k, pad, stride, dil):
+    _conv(dev, orc, N, H, W, C, Co, k, pad, stride, dil)
+
+
+def _conv(dev, orc, N, H, W, C, Co, k, pad, stride, dil, route=None):
     import torch
     from forge_amd import ops
     rng = np.random.default_rng(H * W + C + Co)
@@ -62,7 +66,7 @@ def test_ring_conv(dev, orc, N, H, W, C, Co, k, pad, stride, dil):
     xd, wd = to_dev(x, dev), to_dev(w, dev)
     args = ((pad, pad), (stride, stride), (dil, dil))
     assert np.array_equal(to_host(ops.int8_conv2d_nhwc_s32(xd, wd, *args)), ref)
-    assert ops.last_route().startswith("dma")
+    assert ops.last_route().startswith("dma") if route is None else ops.last_route() == route
     acc = ref.reshape(-1, Co)
     act = rng.uniform(0.001, 0.05, acc.shape[0]).astype(np.float32)
     ws = rng.uniform(0.001, 0.05, Co).astype(np.float16)
@@ -72,6 +76,30 @@ def test_ring_conv(dev, orc, N, H, W, C, Co, k, pad, stride, dil):
     ops.int8_conv2d_nhwc_dequant(xd, wd, to_dev(act, dev), to_dev(ws, dev), to_dev(b, dev), *args, out=Y)
     assert np.array_equal(to_host(Y).reshape(-1, Co).view(np.uint16),
                           orc.dequant_epilogue(acc, act, ws, b).view(np.uint16))
+
+
+# Every tile shape of both gathers at 9 and 10 stages, which starts the K loop of seven XCDs in mid-K and
+# refills every slot: C % 128 == 0 (a stage is one tap), then chunks of 48 channels (a stage straddles
+# taps). Ragged rows and columns, padding, strides and dilations.
+@pytest.mark.parametrize("N,H,W,C,Co,k,pad,stride,dil,route", [
+    (1, 22, 16, 128, 28, 3, 0, 2, 2, "dma64x64"), (8, 40, 29, 128, 65, 3, 0, 1, 1, "dma64x128"),
+    (10, 82, 53, 128, 130, 3, 1, 2, 1, "dma64x192"), (11, 81, 59, 128, 65, 3, 1, 1, 2, "dma128x128"),
+    (7, 25, 86, 128, 65, 3, 2, 1, 1, "dma128x128"), (4, 83, 50, 128, 129, 3, 1, 1, 1, "dma192x128"),
+    (8, 78, 43, 128, 129, 3, 0, 1, 1, "dma128x192"), (7, 84, 87, 128, 391, 3, 0, 2, 1, "dma128x256"),
+    (7, 71, 66, 128, 129, 3, 1, 1, 1, "dma192x192"), (11, 83, 36, 128, 193, 3, 1, 1, 1, "dma192x256"),
+    (10, 72, 73, 128, 129, 3, 0, 1, 1, "dma256x192"), (5, 82, 57, 128, 385, 3, 2, 1, 1, "dma256x256"),
+    (6, 50, 55, 1024, 577, 1, 0, 1, 1, "dma256x256"), (6, 50, 55, 896, 577, 1, 0, 1, 1, "dma192x128"),
+    (2, 9, 7, 256, 40, 16, 9, 1, 1, "dma64x64"),
+    (1, 1, 1, 128, 24, 3, 1, 1, 1, "dma64x64"),         # one pixel in a window of nine: offsets past the image's end
+    (1, 15, 15, 48, 33, 5, 0, 2, 2, "dma64x64"), (4, 49, 46, 48, 65, 5, 1, 1, 1, "dma64x128"),
+    (9, 86, 59, 48, 131, 5, 1, 2, 1, "dma64x192"), (9, 62, 89, 48, 65, 5, 2, 1, 1, "dma128x128"),
+    (10, 76, 27, 48, 65, 5, 0, 1, 1, "dma128x128"), (5, 63, 60, 48, 129, 5, 2, 1, 2, "dma192x128"),
+    (10, 90, 38, 48, 131, 5, 0, 1, 2, "dma128x192"), (4, 46, 89, 48, 390, 5, 0, 1, 2, "dma128x256"),
+    (5, 68, 52, 48, 258, 5, 1, 1, 1, "dma192x192"), (7, 84, 63, 48, 196, 5, 2, 1, 2, "dma192x256"),
+    (11, 35, 70, 48, 262, 5, 1, 1, 1, "dma256x192"), (1, 20, 20, 128, 24, 17, 8, 1, 1, "dma64x64"),
+])
+def test_ring_conv_shapes(dev, orc, N, H, W, C, Co, k, pad, stride, dil, route):
+    _conv(dev, orc, N, H, W, C, Co, k, pad, stride, dil, route)
 
 
 def test_conv_very_wide_kernel(dev, orc):
