@@ -989,7 +989,9 @@ static int launch_sparse_dma(const int8_t* W, const int8_t* X, const uint32_t* m
 // v_smfmac_i32_16x16x128_i8 per stage.
 // BNW = 64 (64 weight rows x 64 tokens, 13 KB stages): twice the tiles, and with a shallower
 // ring two or three workgroups per CU, for the shapes whose 128-row tiles leave CUs idle.
-template <int D, int BNW_ = 128>
+// HALF: K % 128 = 64, the last stage half past K. A template flag, as its selects on every DMA cost whole
+// stages 5-7 % (242 x 8064 x 656 21.1 -> 22.4 us).
+template <int D, int BNW_ = 128, bool HALF = false>
 struct SpRingTile {
     static constexpr int BNW = BNW_, BMT = 64;
     static constexpr int kTN = BNW / 32, kTM = 2;
@@ -1020,7 +1022,7 @@ struct SpRingTile {
             for (int j = 0; j < kTM; j++) acc[i][j] = v4i{0, 0, 0, 0};
 
         const SpBufs bf = sp_bufs(W, X, meta, M, N, K);
-        // K % 128 = 64: the last stage is half past K. Tokens there read as zeros (offsets moved out of
+        // HALF: tokens in the last stage's second half read as zeros (offsets moved out of
         // range), so what the other half of the weights and index words hold adds nothing; those too
         // are moved out of range, which at the last row is the buffer's end.
         uint32_t ow[kWIns], ox[kXIns];
@@ -1050,12 +1052,12 @@ struct SpRingTile {
             oi = static_cast<uint32_t>(b) * cpr * 64 + 16 * (s & 15);
             ti = (s & 15) >= 8;
         }
-        const int nst = (K + 127) / 128;
+        const int nst = HALF ? (K + 127) / 128 : K / 128;
         auto slot_of = [&](int st) { return lds + (st % D) * kSlotBytes; };
         auto issue = [&](int st) {
             int8_t* slot = slot_of(st);
             const uint32_t su = static_cast<uint32_t>(st);
-            const bool half = (st + 1) * 128 > K;
+            const bool half = HALF && (st + 1) * 128 > K;
 #pragma unroll
             for (int q = 0; q < kWIns; q++) dma16_buf(bf.w, half && tw[q] ? 0xC0000000u : ow[q], su * 64, slot + (wave * kWIns + q) * 1024);
 #pragma unroll
@@ -1112,12 +1114,12 @@ constexpr int kSpRingSlots = 8;
 
 // Lane l of block (i, j) holds outputs (m = 16 j + l % 16, n = 16 i + 4 (l / 16) + e): one
 // 8-byte FP16 or 16-byte INT32 store each (N % 16 == 0, so the 4 columns are in or out together).
-template <bool DEQUANT, int BNW = 128, int D = kSpRingSlots>
+template <bool DEQUANT, int BNW = 128, int D = kSpRingSlots, bool HALF = false>
 __global__ __launch_bounds__(256) void sparse_ring_kernel(const int8_t* __restrict__ W, const int8_t* __restrict__ X,
                                                           const uint32_t* __restrict__ meta, GemmEpilogue ep,
                                                           int tiles_n, int tiles_m, int K)
 {
-    using T = SpRingTile<D, BNW>;
+    using T = SpRingTile<D, BNW, HALF>;
     extern __shared__ __align__(16) int8_t lds[];
     int tn, tm;
     tile_coords(blockIdx.x, tiles_n, tiles_m, tn, tm);
@@ -1154,7 +1156,7 @@ __global__ __launch_bounds__(256) void sparse_ring_kernel(const int8_t* __restri
     }
 }
 
-template <bool DEQUANT, int BNW = 128, int D = kSpRingSlots>
+template <bool DEQUANT, int BNW = 128, int D = kSpRingSlots, bool HALF = false>
 static int launch_sparse_ring(const int8_t* W, const int8_t* X, const uint32_t* meta, const GemmEpilogue& ep, int K,
                               hipStream_t s)
 {
@@ -1163,10 +1165,10 @@ static int launch_sparse_ring(const int8_t* W, const int8_t* X, const uint32_t* 
     const int tiles_n = divup(ep.N, T::BNW), tiles_m = divup(ep.M, T::BMT);
     const long long total = static_cast<long long>(tiles_n) * tiles_m;
     if (total > 0x7FFFFFFFLL) return FORGE_EINVAL;
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&sparse_ring_kernel<DEQUANT, BNW, D>),
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&sparse_ring_kernel<DEQUANT, BNW, D, HALF>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     if (attr != hipSuccess) return static_cast<int>(attr);
-    sparse_ring_kernel<DEQUANT, BNW, D>
+    sparse_ring_kernel<DEQUANT, BNW, D, HALF>
         <<<static_cast<unsigned>(total), 256, lds, s>>>(W, X, meta, ep, tiles_n, tiles_m, K);
     return launch_status();
 }
@@ -1414,8 +1416,8 @@ int sparse_gemm(const int8_t* W_comp, const int8_t* x, const uint32_t* meta, con
         void* o = out16 ? static_cast<void*>(out16) : static_cast<void*>(out32);
         GemmEpilogue ep{out32, out16, act_scale, w_scale, bias, M, N, aligned(o, 16) ? 1 : 0};
         note_route("ring64x64");
-        return out16 ? launch_sparse_ring<true, kSpRingRows, kSpRingDepth>(W_comp, x, meta, ep, K, s)
-                     : launch_sparse_ring<false, kSpRingRows, kSpRingDepth>(W_comp, x, meta, ep, K, s);
+        return out16 ? launch_sparse_ring<true, kSpRingRows, kSpRingDepth, true>(W_comp, x, meta, ep, K, s)
+                     : launch_sparse_ring<false, kSpRingRows, kSpRingDepth, true>(W_comp, x, meta, ep, K, s);
     }
     p.split_k = 1;
     p.steps_per_split = steps;
