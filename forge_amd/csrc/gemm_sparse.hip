@@ -1405,14 +1405,19 @@ int sparse_gemm(const int8_t* W_comp, const int8_t* x, const uint32_t* meta, con
         return out16 ? launch_sparse_dma<128, true>(W_comp, x, meta, ep, K, s)
                      : launch_sparse_dma<128, false>(W_comp, x, meta, ep, K, s);
     }
-    // K % 128 = 64: the ring engine, whose last stage is then half zeros, up to one round of its
-    // tiles or 24 stages; deep and large the register-staged 256 x 128 tiles read less. Linear
-    // layers, us, register-staged / ring: 1024 x 5184 x 1280 41.6 / 27.3, 150 x 2368 x 1664 20.7 /
-    // 12.9, 20000 x 2112 x 960 136 / 114, 43057 x 448 x 1728 235 / 158; beyond the line
-    // 2000 x 4160 x 4096 67 / 78, 8192 x 4160 x 8192 470 / 502.
-    const long long ring_tiles = static_cast<long long>(divup(N, kSpRingRows)) * divup(M, 64);
+    // K % 128 = 64: the ring engine, whose last stage is then half zeros, up to one round of its tiles
+    // (3 a CU) at any depth and up to two at 24 stages. Beyond two, against the register-staged tiles that the
+    // planner would take (us, theirs / ring): with FP16 outputs at 24 stages where those are 256 x 128 (linear
+    // layers 20000 x 2112 x 960 136 / 114, 43057 x 448 x 1728 235 / 158, 16451 x 2368 x 1952 215 / 175), at 14
+    // where they are 128 x 128, which read as little (3934 x 2240 x 5040 94 / 106); INT32 outputs, which its
+    // 64-column tiles store in short rows, at 4 and 3 (4447 x 448 x 3136 25.5 / 22.2, but 10503 x 2112 x
+    // 2704 104 / 121, 11547 x 576 x 1408 25.3 / 29.2, 11960 x 1984 x 608 25.7 / 34.6). Past 24 stages
+    // 2000 x 4160 x 4096 67 / 78.
+    const long long ring_w = divupll(static_cast<long long>(divup(N, kSpRingRows)) * divup(M, 64), cu_count_or_default());
+    const bool wide = pt == FORGE_SPARSE_TILE_256x128;
+    const int ring_steps = ring_w <= 2 * kSpRingPerCu ? 24 : out16 ? (wide ? 24 : 14) : (wide ? 4 : 3);
     if (dma_fits && M > 64 && tile == FORGE_SPARSE_TILE_AUTO && static_cast<long long>(N) * K < (1LL << 31) &&
-        (steps <= 24 || ring_tiles <= static_cast<long long>(kSpRingPerCu) * cu_count_or_default())) {
+        (ring_w <= kSpRingPerCu || steps <= ring_steps)) {
         void* o = out16 ? static_cast<void*>(out16) : static_cast<void*>(out32);
         GemmEpilogue ep{out32, out16, act_scale, w_scale, bias, M, N, aligned(o, 16) ? 1 : 0};
         note_route("ring64x64");

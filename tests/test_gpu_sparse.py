@@ -360,3 +360,26 @@ def test_sparse_half_stage(dev, orc, M, K, N, route):
                              split_k=0, out=Y)
         assert ops.last_route().startswith(route)
         assert np.array_equal(to_host(Y).view(np.uint16), orc.dequant_epilogue(ref, act, ws, bias).view(np.uint16))
+
+
+# Past two rounds of ring tiles the outputs and the depth decide.
+@pytest.mark.parametrize("M,K,N,route32,route16", [(20500, 448, 352, "regstaged", "ring64x64"), (20500, 320, 352, "ring64x64", "ring64x64"),
+                                                   (4000, 2240, 5040, "regstaged", "regstaged"), (900, 2240, 2000, "ring64x64", "ring64x64"),
+                                                   (4447, 448, 3136, "ring64x64", "ring64x64")])
+def test_sparse_half_stage_routes(dev, orc, M, K, N, route32, route16):
+    import torch
+    from forge_amd import ops
+    rng = np.random.default_rng(M + K + N)
+    W, x = int8_uniform(rng, (N, K)), int8_uniform(rng, (M, K))
+    act = rng.uniform(0.001, 0.05, M).astype(np.float32)
+    ws = rng.uniform(0.001, 0.05, N).astype(np.float16)
+    cr, mr = orc.prune_compress_24(W)
+    ref = orc.sparse_gemm_s32(cr, x, mr, N, K, threads=orc.cpu_threads())
+    comp, raw, meta = _prep(dev, W)
+    say(f"sparse half stage routes M={M} K={K} N={N}")
+    xd = to_dev(x, dev)
+    assert np.array_equal(to_host(ops.sparse_int8_gemm_s32(comp, xd, meta)), ref)
+    assert ops.last_route().startswith(route32)
+    Y = ops.sparse_int8_gemm(comp, xd, meta, to_dev(act, dev), to_dev(ws, dev), None, split_k=0)
+    assert ops.last_route().startswith(route16)
+    assert np.array_equal(to_host(Y).view(np.uint16), orc.dequant_epilogue(ref, act, ws, None).view(np.uint16))
