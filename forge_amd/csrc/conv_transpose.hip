@@ -29,7 +29,7 @@ namespace forge_amd {
 
 static size_t up256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
 
-// Single-pass kernel for C_in = 32 * KC (KC = 1 .. 8), H*W % 8 == 0: one workgroup (2 waves)
+// Single-pass kernel for C_in = 32 * KC (KC = 1 .. 8; convt_one_pass), H*W % 8 == 0: one workgroup (2 waves)
 // takes 32 consecutive pixels of one image and writes their whole (C_out, 2x2) output, so the
 // INT8 activations never leave the chip and the input is read once. Tiles of 32 pixels (one MFMA
 // row block) rather than 64 give twice the workgroups, whose load, compute and store phases then
@@ -293,6 +293,26 @@ extern "C" size_t forge_int8_conv_transpose2d_k2s2_workspace_size(int C_in, int 
     return M * K * 2 + M * K + M * 4 + Ng * 2 + M * Ng * 2;
 }
 
+// Whether the one-pass kernel takes a layer of one of its channel counts. A workgroup walks all output
+// channels of its 32 pixels, so few pixels of many channels leave most CUs idle where the two kernels
+// spread over the columns: between the powers of two it needs 160 output channels at most or 3 workgroups
+// to 4 CUs (us, two kernels / one pass: (1,160,12,8) -> 504 11.5 / 25.1, (1,192,70,8) -> 224 11.4 / 14.4,
+// (2,96,140,16) -> 376 14.9 / 20.4, but (1,160,65,64) -> 504 30.3 / 27.3, (1,192,19,16) -> 160 11.1 / 11.4,
+// (2,224,4,32) -> 160 12.3 / 11.6). 32, 64, 128 and 256 go as they did.
+static bool convt_one_pass(int N, int C_in, long long HW, int C_out)
+{
+    switch (C_in) {
+        case 32: case 64: case 128: case 256: return true;
+        case 96: case 160: case 192: case 224: break;
+        default: return false;
+    }
+    int st = FORGE_OK;
+    const DeviceInfo& d = device_info(&st);
+    const int cu = st == FORGE_OK && d.cu_count > 0 ? d.cu_count : default_cu_count();
+    const long long groups = N * divupll(HW, 32);
+    return groups < (1 << 25) && (C_out <= 160 || 4 * groups >= 3LL * cu);   // 128 threads a group: the grid's limit
+}
+
 extern "C" int forge_int8_conv_transpose2d_k2s2_forward(const uint16_t* input, const int8_t* weight,
                                                         const uint16_t* w_scale, const uint16_t* bias,
                                                         uint16_t* output, int N, int C_in, int H, int W,
@@ -304,8 +324,9 @@ extern "C" int forge_int8_conv_transpose2d_k2s2_forward(const uint16_t* input, c
     if (HW > 0x7FFFFFFFLL || 4LL * C_out > 0x7FFFFFFFLL) return FORGE_EINVAL;
     hipStream_t s = as_stream(stream);
     if (HW % 8 == 0 && 8LL * C_out * HW < (1LL << 31) && aligned(input, 16) && aligned(weight, 16) &&
-        aligned(output, 4)) {
+        aligned(output, 4) && convt_one_pass(N, C_in, HW, C_out)) {
         const int hw = static_cast<int>(HW);
+        note_route("convt-one-pass");
         switch (C_in) {
             case 32: return launch_convt_fused<1>(input, weight, w_scale, bias, output, N, hw, W, C_out, s);
             case 64: return launch_convt_fused<2>(input, weight, w_scale, bias, output, N, hw, W, C_out, s);

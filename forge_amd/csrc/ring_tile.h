@@ -113,8 +113,8 @@ struct RingConv : ConvGeom {
 // The same gather with C % 128 == 0 and kH, kW <= 16: a stage is 128 channels of one tap, which is
 // uniform, so a lane keeps its pixel's offset and which kernel rows and columns fall inside the image,
 // and a stage costs it a bit test; the position is advanced, not divided. With RingConv's two divisions
-// per DMA instruction, us, RingConv / here: 256 -> 256 3x3 on 33 maps of 36 x 92 98 / 79, 2048 -> 2048 3x3
-// at 92 x 70 266 / 225, over 300 shapes 10 % less; and its lane state, twice this one's, does not fit beside
+// per DMA instruction, us, RingConv / here: 256 -> 256 3x3 on 33 maps of 36 x 92 102 / 72, 2048 -> 2048 3x3
+// at 92 x 70 274 / 216, over 300 shapes 10 % less; and its lane state, twice this one's, does not fit beside
 // the 256 x 256 tile's accumulators. Offsets are taken from `lead` bytes before the image, where the
 // first tap of the first pixel lies, so that none is negative; the resource ends 2 lead past the image,
 // so that it is longer than any scalar offset (a tap outside the image is out of the lane offset's range).
@@ -294,7 +294,7 @@ constexpr int ring_lds_bytes() {
 // 2 c). Column pair (co, kh), kw = 0 and 1, is one 4-byte word and two adjacent outputs of row
 // 2 h + kh; pbias: post_bias per column. vec_out (W % 4 == 0): groups of 4 pixels of one image row
 // go out as one 16-byte store. A lane keeps one group, whose place in the image it finds once (with the
-// two divisions at every word, 16 channels at 56 x 221 -> 111 took 20.4 us, 15.1 so), and walks the pairs;
+// two divisions at every word, 16 channels at 56 x 221 -> 111 took 20.4 us, 12.4 so), and walks the pairs;
 // the LDS words of a batch are all read before its first store.
 template <int kRows, int kCols>
 __device__ __forceinline__ void ring_flush_up2x2(const int8_t* stage, int pitch, const uint16_t* pbias,

@@ -290,3 +290,21 @@ def test_conv_transpose_padded_rows(dev, orc, C_in, N, H, W, C_out, bias):
     y = to_host(ops.int8_conv_transpose2d_k2s2_forward(to_dev(x, dev), to_dev(w, dev), to_dev(ws, dev),
                                                        None if b is None else to_dev(b, dev)))
     assert _bits_equal(y, orc.conv_transpose2d_k2s2(x, w, ws, b))
+
+
+@pytest.mark.parametrize("N,C_in,H,W,C_out,route", [
+    (1, 96, 3, 8, 161, "dma64x64 scatter"), (1, 224, 3, 8, 160, "convt-one-pass"), (2, 192, 5, 24, 200, "dma64x64 scatter"),
+    (1, 160, 75, 80, 170, "dma128x128 scatter"), (1, 160, 77, 80, 170, "convt-one-pass"),     # 188 and 193 workgroups
+    (1, 64, 3, 8, 200, "convt-one-pass")])
+def test_conv_transpose_few_pixels(dev, orc, N, C_in, H, W, C_out, route):
+    """Few pixels of many output channels take the two kernels between the powers of two."""
+    from forge_amd import ops
+    rng = np.random.default_rng(C_in + C_out)
+    x = rng.uniform(-2, 2, (N, C_in, H, W)).astype(np.float16)
+    w = rng.integers(-127, 128, (4 * C_out, C_in)).astype(np.int8)
+    ws = rng.uniform(1e-3, 2e-2, C_out).astype(np.float16)
+    b = rng.uniform(-0.5, 0.5, C_out).astype(np.float16)
+    say(f"conv_transpose few pixels N={N} C_in={C_in} H={H} W={W} C_out={C_out}")
+    y = to_host(ops.int8_conv_transpose2d_k2s2_forward(to_dev(x, dev), to_dev(w, dev), to_dev(ws, dev), to_dev(b, dev)))
+    assert ops.last_route() == route
+    assert _bits_equal(y, orc.conv_transpose2d_k2s2(x, w, ws, b))
