@@ -1193,11 +1193,15 @@ extern "C" int forge_int8_conv2d_forward(const uint16_t* input, const int8_t* we
                              strideH, strideW, dilH, dilW, Ho, Wo};
     // From 48 input channels on, and 48 output channels or 4096 pairs, the NCHW-window kernel below
     // reads its 16-tap chunks and weights too slowly (us, it / conv_deep: 144 -> 32 at 167 x 376
-    // 62 / 25, 64 -> 64 at 134 x 201 33 / 20, 96 -> 96 at 100 x 101 28 / 25, 128 -> 64 at 60 x 80
-    // 17.1 / 16.3); smaller layers (128 -> 32) and few pixels (80 -> 80, 340 pixels: 13.9 / 16.9) stay
-    // on it.
-    if (C_in >= 48 && (C_out >= 48 || static_cast<long long>(C_in) * C_out > 4096) &&
-        static_cast<long long>(N) * M >= 4096) {
+    // 62 / 25, 64 -> 64 at 134 x 201 33 / 20, 96 -> 96 at 100 x 101 28 / 25); smaller layers (128 -> 32)
+    // and few pixels (80 -> 80, 340 pixels: 13.9 / 16.9) stay on it. So do calls of under 16000 pixels and
+    // 0.8 G multiply-adds where its window loads are 16 bytes wide (W % 8 == 0): conv_deep's two launches
+    // are then most of its time (64 -> 128 at 23 x 240 12.1 / 14.8, 72 -> 128 2x2 on two 59 x 56 9.7 /
+    // 14.1, 96 -> 64 at 162 x 344 / 2 14.0 / 17.4; past the line 96 -> 64 at 38 x 408 22.7 / 14.8, 64 -> 96 at
+    // 278 x 72 21.5 / 13.4).
+    const long long pixels = static_cast<long long>(N) * M;
+    if (C_in >= 48 && (C_out >= 48 || static_cast<long long>(C_in) * C_out > 4096) && pixels >= 4096 &&
+        (W % 8 != 0 || !aligned(input, 16) || pixels >= 16000 || static_cast<double>(pixels) * K * C_out >= 0.8e9)) {
         const int r = launch_conv_deep(deep, workspace, ws_bytes, s);
         if (r != -1) return r;
     }

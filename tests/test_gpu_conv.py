@@ -334,7 +334,7 @@ def test_conv_nchw_deep_special_values(dev, orc, W):
     from forge_amd import ops
     from helpers import special_fp16_rows
     rng = np.random.default_rng(78)
-    N, C, H, Co = 2, 64, 27, 160
+    N, C, H, Co = 2, 64, 27, 240     # more weights than the NCHW-window kernel's LDS
     x = special_fp16_rows(rng, N * C * H, W).reshape(N, C, H, W)
     x[1, :, 4:7, 10:20] = 0
     w = int8_uniform(rng, (Co, C * 9))
@@ -349,6 +349,24 @@ def test_conv_nchw_deep_special_values(dev, orc, W):
     y1 = to_host(ops.int8_conv2d_forward(buf[1:].view(N, C, H, W), to_dev(w, dev), to_dev(ws, dev), to_dev(b, dev), 3, 3,
                                          (1, 1)))
     assert np.array_equal(y1.view(np.uint16), y.view(np.uint16))
+
+
+# The line between the NCHW-window kernel and "conv-nchw-deep": pixels and multiply-adds at 16-byte window
+# loads, pixels alone at 2-byte ones, channels.
+@pytest.mark.parametrize("N,C,H,W,Co,route", [
+    (1, 64, 23, 240, 128, "conv-nchw-fused"), (1, 64, 125, 128, 80, "conv-nchw-deep"), (1, 64, 124, 128, 80, "conv-nchw-fused"),
+    (1, 96, 38, 408, 64, "conv-nchw-deep"), (1, 64, 23, 244, 128, "conv-nchw-deep"), (1, 64, 15, 244, 128, "conv-nchw-fused"),
+    (1, 128, 64, 256, 32, "conv-nchw-fused")])
+def test_conv_nchw_deep_line(dev, orc, N, C, H, W, Co, route):
+    rng = np.random.default_rng(H + W + Co)
+    x = rng.uniform(-1, 1, (N, C, H, W)).astype(np.float16)
+    w = int8_uniform(rng, (Co, C * 9))
+    ws = rng.uniform(0.005, 0.05, Co).astype(np.float16)
+    b = rng.uniform(-0.5, 0.5, Co).astype(np.float16)
+    say(f"conv nchw deep line N={N} C={C} H={H} W={W} Co={Co}")
+    y, got = _nchw_run(dev, x, w, ws, b, 3, 1, 1, 1)
+    assert got.startswith(route), got
+    _nchw_check(orc, y, x, w, ws, b, 3, 1, 1, 1)
 
 
 @pytest.mark.parametrize("offset", [1, 2, 8, 15])
