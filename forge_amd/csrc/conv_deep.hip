@@ -28,6 +28,7 @@
 
 #include <algorithm>
 #include <climits>
+#include <cstdio>
 
 namespace forge_amd {
 
@@ -49,7 +50,7 @@ struct ConvDeepArgs {
     uint16_t* y;
     int C, H, W, Co, kH, kW, padH, padW, sH, sW, dH, dW, Ho, Wo;
     int nc, ntg, taps;            // 32-channel chunks; tap groups per chunk; taps
-    int R, Wt, npix, IH, G, IWr;  // tile rows / columns / pixels; window rows; 8-column groups; row pitch (positions)
+    int R, Wt, npix, G, IWr;      // tile rows / columns / pixels; 8-column groups; row pitch (positions)
     int nload;                    // window loads of a chunk (4 channels x 8 columns each)
     int win_bytes, slot_bytes;    // one window buffer, one weight slot
     int tiles_h, tiles_w, tiles;  // tiles per image
@@ -390,12 +391,12 @@ static int launch_deep_kernel(const ConvDeepArgs& a, int images, int groups_co, 
 }
 
 template <int NCB>
-static int launch_deep(const ConvDeepArgs& a, bool al, int images, int groups_co, int waves, int lds, hipStream_t s)
+static int launch_deep(const ConvDeepArgs& a, bool al, int items, int images, int groups_co, int waves, int lds, hipStream_t s)
 {
-    if (a.nload <= 64 * waves)
+    if (items == 1)
         return al ? launch_deep_kernel<NCB, true, 1>(a, images, groups_co, waves, lds, s)
                   : launch_deep_kernel<NCB, false, 1>(a, images, groups_co, waves, lds, s);
-    if (a.nload <= 128 * waves)
+    if (items == 2)
         return al ? launch_deep_kernel<NCB, true, 2>(a, images, groups_co, waves, lds, s)
                   : launch_deep_kernel<NCB, false, 2>(a, images, groups_co, waves, lds, s);
     return al ? launch_deep_kernel<NCB, true, 4>(a, images, groups_co, waves, lds, s)
@@ -462,7 +463,6 @@ int launch_conv_deep(const ConvDeepShape& c, void* workspace, size_t ws_bytes, h
                     lds = static_cast<int>(bytes);
                     a.Wt = wt;
                     a.R = R;
-                    a.IH = static_cast<int>(IH);
                     a.G = static_cast<int>(G);
                     a.nload = static_cast<int>(nload);
                     a.win_bytes = static_cast<int>(win);
@@ -505,7 +505,10 @@ int launch_conv_deep(const ConvDeepShape& c, void* workspace, size_t ws_bytes, h
     a.wf = wf;
     a.amax = amax;
     const bool al = c.W % 8 == 0 && aligned(c.x, 16);
-    note_route("conv-nchw-deep", 32 * waves);
+    const int items = a.nload <= 64 * waves ? 1 : a.nload <= 128 * waves ? 2 : 4;
+    char name[32];
+    snprintf(name, sizeof name, "conv-nchw-deep b%d i%d%s", ncb, items, al ? " a" : "");
+    note_route(name, 32 * waves);
     for (int n0 = 0; n0 < c.N; n0 += static_cast<int>(chunk)) {
         const int cnt = static_cast<int>(std::min<long long>(chunk, c.N - n0));
         a.x = c.x + static_cast<size_t>(n0) * c.C * HW;
@@ -517,10 +520,10 @@ int launch_conv_deep(const ConvDeepShape& c, void* workspace, size_t ws_bytes, h
             a.x, amax, c.w, wf, c.C, static_cast<int>(HW), groups, cnt, mblocks, c.Co, taps, a.nc, ncb, nfrag);
         if ((st = launch_status()) != FORGE_OK) return st;
         switch (ncb) {
-            case 1: st = launch_deep<1>(a, al, cnt, groups_co, waves, lds, s); break;
-            case 2: st = launch_deep<2>(a, al, cnt, groups_co, waves, lds, s); break;
-            case 3: st = launch_deep<3>(a, al, cnt, groups_co, waves, lds, s); break;
-            default: st = launch_deep<4>(a, al, cnt, groups_co, waves, lds, s); break;
+            case 1: st = launch_deep<1>(a, al, items, cnt, groups_co, waves, lds, s); break;
+            case 2: st = launch_deep<2>(a, al, items, cnt, groups_co, waves, lds, s); break;
+            case 3: st = launch_deep<3>(a, al, items, cnt, groups_co, waves, lds, s); break;
+            default: st = launch_deep<4>(a, al, items, cnt, groups_co, waves, lds, s); break;
         }
         if (st != FORGE_OK) return st;
     }

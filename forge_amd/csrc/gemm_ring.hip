@@ -194,7 +194,7 @@ static int launch_ring_tail(const RingRowMajor& opa, const RingRowMajor& opb, co
 static void note_shape(int shape)
 {
     char name[24];
-    snprintf(name, sizeof name, "dma%dx%d", kShapes[shape].bm, kShapes[shape].bn);
+    snprintf(name, sizeof name, "dma%dx%d%s", kShapes[shape].bm, kShapes[shape].bn, shape == k128x128deep ? " 4-slot" : "");
     note_route(name);
 }
 

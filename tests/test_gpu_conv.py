@@ -43,12 +43,12 @@ def test_conv_random(dev, orc, N, H, W, C, Co, k, pad, stride, dil):
     assert np.array_equal(to_host(out), ref)
 
 
-# C % 128 == 0 with grids large enough for the DMA engine (128- and 256-row tiles): the
-# implicit-im2col gather by DMA, padding read from the zero line, ragged last tile.
+# C % 128 == 0: the ring tiles' gather of whole taps, padding read as zeros past the image's range, ragged
+# last tile (the first shape on the window-fed tile, whose rows it fills).
 @pytest.mark.parametrize("N,H,W,C,Co,k,pad,stride,dil,check", [
-    (2, 64, 64, 128, 256, 3, 1, 1, 1, "all"),      # 128x128 tiles, padding
+    (2, 64, 64, 128, 256, 3, 1, 1, 1, "all"),      # padding
     (2, 63, 61, 128, 384, 3, 1, 1, 1, "all"),      # ragged rows (7686)
-    (8, 130, 130, 128, 256, 3, 2, 2, 2, "ends"),   # 256x256 tiles, stride 2, dilation 2
+    (8, 130, 130, 128, 256, 3, 2, 2, 2, "ends"),   # large tiles, stride 2, dilation 2
     (4, 40, 40, 256, 256, 1, 0, 1, 1, "all"),      # pointwise, two stages per tap
 ])
 def test_conv_dma_gather(dev, orc, N, H, W, C, Co, k, pad, stride, dil, check):
@@ -324,6 +324,52 @@ def test_conv_nchw_deep(dev, orc, N, C, H, W, Co, k, pad, stride, dil, bias):
     say(f"conv nchw deep N={N} C={C} H={H} W={W} Co={Co} k={k} s={stride} d={dil}")
     y, route = _nchw_run(dev, x, w, ws, b, k, pad, stride, dil)
     assert route.startswith("conv-nchw-deep"), route
+    _nchw_check(orc, y, x, w, ws, b, k, pad, stride, dil)
+
+
+# Every form of the kernel: 1 to 4 blocks of 32 output channels per workgroup, 1, 2 or 4 window loads per
+# lane, aligned and shifted ones, 9 taps (unrolled) and 4 or 25 (a loop); then workgroups of 9 to 12 waves,
+# the layer of 128 -> 128 channels at 135 x 240 among them.
+DEEP_FORMS = [
+    (3, 240, 6, 28, 16, 3, 1, 1, 1, "b1 i1 "), (2, 240, 9, 32, 16, 3, 1, 1, 1, "b1 i1 a"),
+    (3, 240, 14, 9, 16, 3, 2, 1, 2, "b1 i2 "), (2, 96, 10, 15, 16, 5, 2, 1, 1, "b1 i2 "),
+    (2, 240, 16, 8, 16, 3, 1, 1, 1, "b1 i2 a"), (2, 88, 15, 8, 16, 5, 2, 1, 1, "b1 i2 a"),
+    (2, 232, 30, 14, 16, 3, 1, 2, 1, "b1 i4 "), (2, 96, 7, 18, 16, 5, 4, 1, 2, "b1 i4 "),
+    (2, 232, 10, 40, 16, 3, 1, 2, 1, "b1 i4 a"), (2, 96, 6, 80, 16, 5, 2, 2, 1, "b1 i4 a"),
+    (2, 240, 5, 28, 48, 3, 1, 1, 1, "b2 i1 "), (3, 264, 4, 48, 48, 3, 1, 1, 1, "b2 i1 a"),
+    (2, 232, 10, 11, 48, 3, 2, 1, 2, "b2 i2 "), (2, 88, 8, 18, 60, 5, 2, 1, 1, "b2 i2 "),
+    (2, 232, 8, 16, 48, 3, 1, 1, 1, "b2 i2 a"), (2, 88, 4, 32, 48, 5, 2, 1, 1, "b2 i2 a"),
+    (2, 232, 15, 26, 48, 3, 1, 2, 1, "b2 i4 "), (2, 88, 4, 27, 48, 5, 4, 1, 2, "b2 i4 "),
+    (2, 240, 9, 40, 48, 3, 1, 2, 1, "b2 i4 a"), (2, 96, 10, 40, 60, 5, 2, 2, 1, "b2 i4 a"),
+    (2, 264, 8, 14, 72, 3, 1, 1, 1, "b3 i1 "), (3, 232, 4, 48, 72, 3, 1, 1, 1, "b3 i1 a"),
+    (2, 232, 12, 9, 72, 3, 1, 1, 1, "b3 i2 "), (2, 88, 15, 11, 72, 5, 2, 1, 1, "b3 i2 "),
+    (2, 232, 13, 8, 72, 3, 2, 1, 2, "b3 i2 a"), (2, 88, 15, 8, 72, 5, 2, 1, 1, "b3 i2 a"),
+    (2, 232, 8, 58, 72, 3, 1, 2, 1, "b3 i4 "), (2, 88, 8, 30, 72, 5, 4, 1, 2, "b3 i4 "),
+    (2, 232, 9, 40, 72, 3, 1, 2, 1, "b3 i4 a"), (2, 88, 15, 8, 72, 5, 4, 1, 2, "b3 i4 a"),
+    (2, 240, 4, 26, 100, 3, 1, 1, 1, "b4 i1 "), (3, 240, 4, 48, 100, 3, 1, 1, 1, "b4 i1 a"),
+    (2, 240, 11, 9, 120, 3, 1, 1, 1, "b4 i2 "), (2, 88, 11, 10, 120, 5, 2, 1, 1, "b4 i2 "),
+    (2, 240, 13, 8, 100, 3, 2, 1, 2, "b4 i2 a"), (2, 88, 7, 16, 128, 5, 2, 1, 1, "b4 i2 a"),
+    (2, 240, 10, 116, 128, 3, 1, 2, 1, "b4 i4 "), (3, 96, 5, 21, 100, 5, 4, 1, 2, "b4 i4 "),
+    (3, 232, 9, 40, 100, 3, 1, 2, 1, "b4 i4 a"), (2, 88, 6, 24, 120, 5, 4, 1, 2, "b4 i4 a"),
+    (3, 528, 6, 13, 16, 2, 1, 1, 1, "b1 i1 "), (3, 528, 4, 24, 16, 2, 1, 1, 1, "b1 i1 a"),
+    (2, 520, 5, 34, 48, 2, 1, 1, 1, "b2 i1 "), (2, 528, 7, 24, 48, 2, 1, 1, 1, "b2 i1 a"),
+    (2, 528, 9, 18, 96, 2, 1, 1, 1, "b3 i1 "), (3, 520, 6, 16, 96, 2, 1, 1, 1, "b3 i1 a"),
+    (2, 528, 11, 10, 128, 2, 1, 1, 1, "b4 i1 "), (2, 528, 9, 16, 100, 2, 1, 1, 1, "b4 i1 a"),
+    (2, 128, 135, 240, 128, 3, 1, 1, 1, "b4 i1 a tile288"), (3, 96, 53, 198, 200, 3, 1, 1, 1, "b4 i1 tile288"),
+    (2, 232, 148, 216, 16, 3, 1, 1, 1, "b1 i1 a tile288"), (3, 96, 104, 230, 48, 3, 1, 1, 1, "b2 i1 tile320"),
+    (3, 96, 114, 233, 72, 3, 1, 1, 1, "b3 i1 tile352"), (3, 96, 117, 251, 64, 3, 1, 1, 1, "b2 i1 tile384")]
+
+
+@pytest.mark.parametrize("N,C,H,W,Co,k,pad,stride,dil,form", DEEP_FORMS)
+def test_conv_nchw_deep_forms(dev, orc, N, C, H, W, Co, k, pad, stride, dil, form):
+    rng = np.random.default_rng(C * W + Co + k + stride)
+    x = rng.uniform(-1, 1, (N, C, H, W)).astype(np.float16)
+    w = int8_uniform(rng, (Co, C * k * k))
+    ws = rng.uniform(0.005, 0.05, Co).astype(np.float16)
+    b = rng.uniform(-0.5, 0.5, Co).astype(np.float16)
+    say(f"conv nchw deep form N={N} C={C} H={H} W={W} Co={Co} k={k} s={stride} d={dil} {form}")
+    y, route = _nchw_run(dev, x, w, ws, b, k, pad, stride, dil)
+    assert route.startswith("conv-nchw-deep " + form) and (" a" in form) == (" a " in route), route
     _nchw_check(orc, y, x, w, ws, b, k, pad, stride, dil)
 
 

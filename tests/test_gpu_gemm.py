@@ -129,9 +129,8 @@ def test_4096_cube_int32(dev, orc):
 
 @pytest.mark.parametrize("N", [256, 200])
 def test_gemm_tail_split(dev, orc, N):
-    """M = 70,000 rows in one column of 256x256 tiles: 274 tiles, the second wave 7 % full, so
-    the first 65,536 rows run as 256-row tiles and the rest as 192-row tiles in a second
-    launch. Rows on both sides of the boundary and the last rows bit-exact (INT32 and FP16);
+    """M = 70,000 rows of two narrow column tiles (192 x 128, several tiles per CU, the last row tile 112
+    rows): rows on both sides of tile boundaries and the last rows bit-exact (INT32 and FP16);
     every column's sum over all rows equals (sum of A's rows) . B (exact in int64)."""
     import torch
     from forge_amd import ops

@@ -1,7 +1,8 @@
 """GPU parity of the ring-fed tiles: every tile shape of the dense choice (checked by route) at
-ragged rows and columns, K of 1 stage to several and not a multiple of 128, the NHWC gather at
-C % 128 != 0, and the transposed conv's scatter. Integer sums are exact, and the FP16 epilogue is the
-oracle's, so every output is compared bit for bit."""
+ragged rows and columns and K not a multiple of 128, each at one or two stages and at 5 or 9, which
+refill every slot and start the K loop of seven XCDs in mid-K; both NHWC gathers likewise; and the
+transposed conv's scatter. Integer sums are exact, and the FP16 epilogue is the oracle's, so every
+output is compared bit for bit."""
 import numpy as np
 import pytest
 
@@ -12,10 +13,16 @@ pytestmark = pytest.mark.gpu
 SHAPES = [
     (62, 208, 40, "dma64x64"), (700, 1040, 999, "dma64x64"), (131, 544, 5538, "dma64x128"),
     (322, 656, 5565, "dma64x192"), (67, 48, 3, "dma64x64"),
-    (327, 16, 5708, "dma128x128"), (2694, 912, 1001, "dma128x128"),
+    (327, 16, 5708, "dma128x128"), (2694, 912, 1001, "dma128x128 4-slot"),
     (642, 16, 5390, "dma192x128"), (1159, 16, 4652, "dma128x192"), (1033, 144, 5418, "dma128x256"),
     (2315, 144, 3339, "dma192x192"), (2092, 16, 5763, "dma192x256"), (2813, 16, 4392, "dma256x192"),
     (2438, 16, 4888, "dma256x256"), (1030, 400, 13001, "dma256x256"),
+    # at least 2 slots + 1 stages: the loop's partial waits, slot advance and refills
+    (61, 1040, 41, "dma64x64"), (8205, 1040, 65, "dma64x128"), (129, 1040, 10893, "dma64x192"),
+    (8203, 528, 193, "dma128x128"), (8267, 1040, 194, "dma128x128 4-slot"), (10921, 1040, 258, "dma192x128"),
+    (385, 1040, 10916, "dma128x192"), (8209, 1040, 643, "dma128x256"), (11002, 1040, 516, "dma192x192"),
+    (9893, 1040, 769, "dma192x256"), (9796, 1040, 1031, "dma256x192"), (1539, 1040, 7204, "dma256x256"),
+    (1000, 1040, 17900, "dma256x256+tail192"),
 ]
 
 
@@ -84,7 +91,7 @@ def _conv(dev, orc, N, H, W, C, Co, k, pad, stride, dil, route=None):
 @pytest.mark.parametrize("N,H,W,C,Co,k,pad,stride,dil,route", [
     (1, 22, 16, 128, 28, 3, 0, 2, 2, "dma64x64"), (8, 40, 29, 128, 65, 3, 0, 1, 1, "dma64x128"),
     (10, 82, 53, 128, 130, 3, 1, 2, 1, "dma64x192"), (11, 81, 59, 128, 65, 3, 1, 1, 2, "dma128x128"),
-    (7, 25, 86, 128, 65, 3, 2, 1, 1, "dma128x128"), (4, 83, 50, 128, 129, 3, 1, 1, 1, "dma192x128"),
+    (7, 25, 86, 128, 65, 3, 2, 1, 1, "dma128x128 4-slot"), (4, 83, 50, 128, 129, 3, 1, 1, 1, "dma192x128"),
     (8, 78, 43, 128, 129, 3, 0, 1, 1, "dma128x192"), (7, 84, 87, 128, 391, 3, 0, 2, 1, "dma128x256"),
     (7, 71, 66, 128, 129, 3, 1, 1, 1, "dma192x192"), (11, 83, 36, 128, 193, 3, 1, 1, 1, "dma192x256"),
     (10, 72, 73, 128, 129, 3, 0, 1, 1, "dma256x192"), (5, 82, 57, 128, 385, 3, 2, 1, 1, "dma256x256"),
@@ -93,7 +100,7 @@ def _conv(dev, orc, N, H, W, C, Co, k, pad, stride, dil, route=None):
     (1, 1, 1, 128, 24, 3, 1, 1, 1, "dma64x64"),         # one pixel in a window of nine: offsets past the image's end
     (1, 15, 15, 48, 33, 5, 0, 2, 2, "dma64x64"), (4, 49, 46, 48, 65, 5, 1, 1, 1, "dma64x128"),
     (9, 86, 59, 48, 131, 5, 1, 2, 1, "dma64x192"), (9, 62, 89, 48, 65, 5, 2, 1, 1, "dma128x128"),
-    (10, 76, 27, 48, 65, 5, 0, 1, 1, "dma128x128"), (5, 63, 60, 48, 129, 5, 2, 1, 2, "dma192x128"),
+    (10, 76, 27, 48, 65, 5, 0, 1, 1, "dma128x128 4-slot"), (5, 63, 60, 48, 129, 5, 2, 1, 2, "dma192x128"),
     (10, 90, 38, 48, 131, 5, 0, 1, 2, "dma128x192"), (4, 46, 89, 48, 390, 5, 0, 1, 2, "dma128x256"),
     (5, 68, 52, 48, 258, 5, 1, 1, 1, "dma192x192"), (7, 84, 63, 48, 196, 5, 2, 1, 2, "dma192x256"),
     (11, 35, 70, 48, 262, 5, 1, 1, 1, "dma256x192"), (1, 20, 20, 128, 24, 17, 8, 1, 1, "dma64x64"),
