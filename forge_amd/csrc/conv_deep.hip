@@ -50,8 +50,9 @@ struct ConvDeepArgs {
     uint16_t* y;
     int C, H, W, Co, kH, kW, padH, padW, sH, sW, dH, dW, Ho, Wo;
     int nc, ntg, taps;            // 32-channel chunks; tap groups per chunk; taps
-    int R, Wt, npix, G, IWr;      // tile rows / columns / pixels; 8-column groups; row pitch (positions)
+    int R, Wt, npix;              // tile rows / columns / pixels
     int nload;                    // window loads of a chunk (4 channels x 8 columns each)
+    int G, IWr;                   // 8-column groups; row pitch (positions)
     int win_bytes, slot_bytes;    // one window buffer, one weight slot
     int tiles_h, tiles_w, tiles;  // tiles per image
     uint32_t mg_wt, mg_g, mg_tiles, mg_tw;

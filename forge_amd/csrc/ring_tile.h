@@ -206,19 +206,18 @@ struct RingTile {
         const int nst = (K + kBK - 1) / kBK;
         typename OpA::Pos pa = opa.at(rot);          // the stages in order from rot on
         typename OpB::Pos pb = opb.at(rot);
-        auto issue = [&](int st, int slot) {
+        auto dmas = [&](bool live, int slot) {
             int8_t* s = lds + slot * kSlotBytes;
-            const bool live = st < nst;
-            if (st > 0) {
-                st += rot;
-                st = st < nst ? st : st - nst;
-                opa.step(pa, st);
-                opb.step(pb, st);
-            }
 #pragma unroll
             for (int q = 0; q < kAIns; q++) opa.dma(la[q], pa, live, s + (wave * kAIns + q) * 1024);
 #pragma unroll
             for (int q = 0; q < kBIns; q++) opb.dma(lb[q], pb, live, s + BM * kBK + (wave * kBIns + q) * 1024);
+        };
+        auto issue = [&](int st, int slot) {         // stages 1 on
+            const int at = st + rot;
+            opa.step(pa, at < nst ? at : at - nst);
+            opb.step(pb, at < nst ? at : at - nst);
+            dmas(st < nst, slot);
         };
         struct Frags {
             v4i a[kTM], b[kTN];
@@ -241,8 +240,9 @@ struct RingTile {
         };
         constexpr int kMf = kTM * kTN, kRd = kTM + kTN;
 
+        dmas(true, 0);
 #pragma unroll
-        for (int st = 0; st < D; st++) issue(st, st);
+        for (int st = 1; st < D; st++) issue(st, st);
         wait_vmcnt<kIns*(D - 1) < 64 ? kIns * (D - 1) : 63>();
         lds_barrier();
         Frags F[2];
