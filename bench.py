@@ -4,15 +4,15 @@
     python bench.py --traffic-probe     (the dominant kernels, for rocprofv3 --pmc counter runs)
     python bench.py --counter-summary DIR   (rocprofv3 CSVs -> profiles/kernel_counters.{json,md})
 
-Headline (`value`): configs[1] of BASELINE.json -- the fused W8A8 linear at M=N=K=4096
+Headline (`value`): the fused W8A8 linear at M=N=K=4096
 (FP16 activations with 8 outlier channels x20, per-token quantize, INT8 MFMA GEMM with
 INT32 accumulation, dequant + bias to FP16). One step = one forge_int8_linear call
 (quantize kernel + GEMM kernel) on inputs already resident in HBM. value = 2*M*N*K / t.
 
 roofline: the dominant kernel (the GEMM) timed alone with HIP events on the launch stream,
 algorithmic ops 2*M*N*K per launch against MI355X's dense INT8 peak (5.0 POP/s).
-cpu_baseline: the oracle's INT32 loop + dequant epilogue (oracle/) over the whole configs[1]
-workload, split over output rows on up to 16 threads (the box's CPU share per GPU), timed on
+cpu_baseline: the oracle's INT32 loop + dequant epilogue (oracle/) over the whole
+workload, split over output rows on up to 16 threads (a host's CPU share per GPU), timed on
 this host; the single-threaded rate is in its sample text.
 roofline.traffic / roofline.mfma_busy: L2-miss bytes per launch of the GEMM (reads and writes
 between the L2s and the memory fabric: HBM plus what the 256 MB MALL serves, so an upper bound
@@ -20,11 +20,11 @@ of HBM bytes) and its matrix-core busy fraction, read from COUNTERS_FILE (profil
 writes from rocprofv3 --pmc runs of `bench.py --traffic-probe` (FETCH_SIZE and WRITE_SIZE scaled
 by what the same counters read for a device copy of known size in the same runs; MFMA busy
 cycles; see profiles/kernel_counters.md).
-extra: configs[2] (2:4 sparse vs dense at 4096x11008x4096), configs[3] (decode
+extra: 2:4 sparse vs dense at 4096x11008x4096, decode (
 M = 1/4/16, N = K = 8192, dense and 2:4, HBM GB/s with 8 dense / 10 sparse rotating weight
 copies so the 256 MB MALL cannot hold them; calls captured into a HIP graph and replayed so host launch
 overhead is not timed; the whole int8_linear / sparse_int8_linear, and the GEMM alone on
-pre-quantized tokens, *_gemm_*), configs[4] (INT8 NHWC 3x3 conv, INT32 and dequant outputs), and
+pre-quantized tokens, *_gemm_*), INT8 NHWC 3x3 conv (32,56,56,256) (INT32 and dequant outputs), and
 the rest of the INT8 conv family on NCHW FP16 maps: depthwise 3x3 (1, 64, 540, 960) and
 ConvTranspose2d k2s2 (1, 64, 270, 480) -> (1, 32, 540, 960), as time and HBM GB/s of
 input + output bytes (rotating over more than 256 MB of inputs and outputs, graph-replayed); the
@@ -70,7 +70,7 @@ def _c2_counters():
 
 
 def measured_traffic():
-    """L2-miss bytes per launch of the configs[1] GEMM (L2 <-> memory fabric, HBM plus MALL
+    """L2-miss bytes per launch of the 4096^3 GEMM (L2 <-> memory fabric, HBM plus MALL
     hits) from the committed counter runs (FETCH_SIZE and WRITE_SIZE, scaled by the counters'
     reading for a device copy of known size), or None."""
     v = _c2_counters().get("traffic_bytes")
@@ -78,7 +78,7 @@ def measured_traffic():
 
 
 def measured_mfma_busy():
-    """Matrix-core busy fraction of the configs[1] GEMM from the committed counter run
+    """Matrix-core busy fraction of the 4096^3 GEMM from the committed counter run
     (SQ_VALU_MFMA_BUSY_CYCLES over 4 x SQ_BUSY_CU_CYCLES), or None."""
     v = _c2_counters().get("mfma_busy")
     return round(float(v), 4) if v is not None else None
@@ -86,10 +86,10 @@ def measured_mfma_busy():
 
 def traffic_probe() -> int:
     """Launches for the counter runs (rocprofv3 --pmc, one counter set per run), each kernel
-    PROBE_REPS times on its configs' shape with inputs resident on the device:
-    c2 = the configs[1] dequant GEMM (4096^3, FP16 out); c3 sparse / dense = configs[2]
-    (4096 x 11008 x 4096, INT32 out) on the 2:4 and the dense engine; c5 = configs[4] NHWC
-    conv (INT32 out; 256-row and 192-row tiles in one launch); c4 = configs[3] M = 16 decode GEMMs
+    PROBE_REPS times on its shape with inputs resident on the device:
+    c2 = the dequant GEMM (4096^3, FP16 out); c3 sparse / dense = 4096 x 11008 x 4096
+    (INT32 out) on the 2:4 and the dense engine; c5 = the NHWC conv
+    (32,56,56,256) 3x3 (INT32 out, window-fed tiles); c4 = M = 16 decode GEMMs
     (N = K = 8192, pre-quantized tokens, FP16 out) dense and 2:4; f1 = the fused quantize + 2:4
     sparse linear on the reference's example layer (1280 -> 320 at M = 147,456); f2 = the NCHW FP16
     conv API on (1, 32, 540, 960) 3x3 -> 32 (one launch); then a COPY_PROBE_BYTES
@@ -326,12 +326,12 @@ COUNTER_SETS = [
            "TCP_TCC_READ_REQ_LATENCY_sum"),
 ]
 PROBE_TITLES = {
-    "c2_gemm": "configs[1] GEMM 4096^3, FP16 out (`gemm_ring_kernel` on 256x256 tiles)",
-    "c3_sparse": "configs[2] 2:4 sparse 4096x11008x4096, INT32 out (`sparse_wide_s32_kernel`: 256 tokens x 320-352 weight rows per tile, 2 tiles per CU)",
-    "c3_dense": "configs[2] shape dense, INT32 out (`gemm_ring_tail_kernel<false>`: 256- and 192-row tiles, one launch)",
-    "c5_conv": "configs[4] NHWC conv, INT32 out (`conv_window_kernel<7,2,false>`: 224-pixel x 256-channel tiles, input window in LDS once per channel chunk)",
-    "c4_dense_M16": "configs[3] M=16 dense decode GEMM (`decode_dense_kernel`)",
-    "c4_sparse_M16": "configs[3] M=16 2:4 decode GEMM (`decode_sparse_reg_kernel`)",
+    "c2_gemm": "GEMM 4096^3, FP16 out (`gemm_ring_kernel` on 256x256 tiles)",
+    "c3_sparse": "2:4 sparse 4096x11008x4096, INT32 out (`sparse_wide_s32_kernel`: 256 tokens x 320-352 weight rows per tile, 2 tiles per CU)",
+    "c3_dense": "4096x11008x4096 dense, INT32 out (`gemm_ring_tail_kernel<false>`: 256- and 192-row tiles, one launch)",
+    "c5_conv": "NHWC conv (32,56,56,256) 3x3 -> 256, INT32 out (`conv_window_kernel<7,2,false>`: 224-pixel x 256-channel tiles, input window in LDS once per channel chunk)",
+    "c4_dense_M16": "N = K = 8192 M=16 dense decode GEMM (`decode_dense_kernel`)",
+    "c4_sparse_M16": "N = K = 8192 M=16 2:4 decode GEMM (`decode_sparse_reg_kernel`)",
     "f1_fq": "fused quantize + 2:4 sparse linear 1280->320 at M=147,456 (`sparse_fq_kernel<5,48,true,3>`)",
     "f2_conv_nchw": "`int8_conv2d_forward` NCHW FP16 (1,32,540,960) 3x3 -> 32 (`conv_nchw_cl_kernel<1,true,8>`: channel-last window, 256-pixel tiles)",
 }
@@ -342,7 +342,7 @@ def _counter_markdown(out) -> str:
     L = ["# Hardware counters of the dominant kernels (one MI355X)", "",
          "Made by `bench.py --traffic-probe` under `rocprofv3 --pmc`, one counter set per run, then "
          "`python bench.py --counter-summary <out>` (this file and `kernel_counters.json`). Commands, from the "
-         "repository root on the GPU box:", "", "```", "cd /tmp && export TMPDIR=/tmp && cd <repo>"]
+         "repository root:", "", "```", "cd /tmp && export TMPDIR=/tmp && cd <repo>"]
     for name, counters in COUNTER_SETS:
         L.append(f"rocprofv3 --pmc {counters} --output-format csv -d <out>/{name} -o {name} -- "
                  f"python3 bench.py --traffic-probe")
@@ -353,7 +353,7 @@ def _counter_markdown(out) -> str:
           "cycles, a 256-thread fill kernel), taken once per launch.",
           "- MFMA busy = SQ_VALU_MFMA_BUSY_CYCLES / (4 SIMDs x SQ_BUSY_CU_CYCLES): matrix-core busy cycles over "
           "the SIMD cycles of CUs holding waves. The counter adds 32 cycles per `v_mfma_i32_32x32x32_i8` and per "
-          "`v_smfmac_i32_32x32x64_i8` (checked: c2 = 2,097,152 MFMAs x 32); `at clock` divides by 1024 SIMDs x "
+          "`v_smfmac_i32_32x32x64_i8`, 16 per `v_mfma_i32_16x16x64_i8` (checked: c2 = 4,194,304 MFMAs x 16); `at clock` divides by 1024 SIMDs x "
           "clock x duration instead.",
           "- peak at clock = the 2.4 GHz peak (dense INT8 5.0 POP/s, 2:4 10.0) scaled to the measured clock.",
           f"- L2-miss bytes = FETCH_SIZE x {cal['fetch_scale']:.3f} + WRITE_SIZE x {cal['write_scale']:.3f} (KiB x 1024), "
@@ -716,8 +716,8 @@ def make_c2(dev, seed=2):
 
 
 def cpu_baseline(target_s: float = 12.0):
-    """The oracle's INT32 loop + dequant epilogue (oracle/) on configs[1] (M = N = K = 4096),
-    split over output rows on the host's cores up to 16 POSIX threads (the GPU box's CPU share
+    """The oracle's INT32 loop + dequant epilogue (oracle/) on the headline workload (M = N = K = 4096),
+    split over output rows on the host's cores up to 16 POSIX threads (a host's CPU share
     per GPU; nproc is recorded), over the whole workload; the single-threaded rate over as many
     rows as fit in about target_s seconds is recorded in the sample text."""
     from oracle import oracle
@@ -748,10 +748,10 @@ def cpu_baseline(target_s: float = 12.0):
     except OSError:
         pass
     return {"value": tops, "unit": "TOPS", "cores": threads, "kind": "port",
-            "sample": f"oracle INT32 loop + dequant epilogue over all 4096 rows of configs[1] (N=K=4096) split "
+            "sample": f"oracle INT32 loop + dequant epilogue over all 4096 rows (N=K=4096) split "
                       f"over output rows on {threads} threads: {tm:.2f} s; one thread over {rows} rows: "
                       f"{t1:.2f} s = {tops1:.4f} TOPS; gcc -O3, host CPU '{model}', nproc {nproc} (threads capped "
-                      f"at 16, the box's CPU share per GPU)"}
+                      f"at 16, a host's CPU share per GPU)"}
 
 
 def bench_extra(dev):
@@ -760,7 +760,7 @@ def bench_extra(dev):
     out = {}
     g = torch.Generator(device=dev)
     g.manual_seed(3)
-    # configs[2]: 2:4 sparse 4096 x 11008 x 4096 INT32 out, and the same shape dense
+    # 2:4 sparse 4096 x 11008 x 4096 INT32 out, and the same shape dense
     M, K, N = 4096, 4096, 11008
     W = torch.randint(-127, 128, (N, K), generator=g, device=dev, dtype=torch.int8)
     x = torch.randint(-127, 128, (M, K), generator=g, device=dev, dtype=torch.int8)
@@ -794,7 +794,7 @@ def bench_extra(dev):
     del W, x, comp, raw, meta, C
     torch.cuda.empty_cache()
 
-    # configs[3]: decode, N = K = 8192; rotating weight copies so that the 256 MB MALL cannot
+    # decode, N = K = 8192; rotating weight copies so that the 256 MB MALL cannot
     # serve them: 8 dense copies (537 MB), 10 sparse copies (W_comp + index words, 420 MB).
     N = K = 8192
     copies, sp_copies = 8, 10
@@ -842,7 +842,7 @@ def bench_extra(dev):
     del Ws, comps, metas
     torch.cuda.empty_cache()
 
-    # configs[4]: INT8 NHWC conv 3x3, pad 1, stride 1: (32,56,56,256) x (256,3,3,256) -> INT32,
+    # INT8 NHWC conv 3x3, pad 1, stride 1: (32,56,56,256) x (256,3,3,256) -> INT32,
     # and the same with the per-channel dequant + bias epilogue (FP16 out). Implicit GEMM
     # M = 32*56*56 = 100,352, N = 256, K = 2,304.
     xc = torch.randint(-127, 128, (32, 56, 56, 256), generator=g, device=dev, dtype=torch.int8)
@@ -855,7 +855,7 @@ def bench_extra(dev):
     o16 = torch.empty((32, 56, 56, 256), dtype=torch.float16, device=dev)
     conv32 = lambda: ops.int8_conv2d_nhwc_s32(xc, wc, pad=(1, 1), out=o32)
     conv16 = lambda: ops.int8_conv2d_nhwc_dequant(xc, wc, asc, wsc, bc, pad=(1, 1), out=o16)
-    spin(lambda: (conv32(), conv16()), 1.0)     # settled clocks, as for configs[2]
+    spin(lambda: (conv32(), conv16()), 1.0)     # settled clocks, as for the sparse pair
     t32 = events_time_ms(conv32, 10)
     t16 = events_time_ms(conv16, 10)
     ops_c = 2.0 * Mc * 256 * 2304
@@ -918,7 +918,7 @@ def bench_extra(dev):
     del xcs, ycs, wspn
     torch.cuda.empty_cache()
 
-    # Weight preparation for SparseLinear at configs[2]'s weight (11008 x 4096, fp32): the one
+    # Weight preparation for SparseLinear at an 11008 x 4096 fp32 weight: the one
     # pass (quantize + prune + compress + gfx950 pack) against the reference's sequence of
     # separate steps (quantize rows, prune_compress_24 through a raw-nibble buffer, pack).
     N, K = 11008, 4096
@@ -1053,9 +1053,9 @@ def main() -> int:
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "int8",
-        "data": "synthetic (configs[1]: N(0,1) fp16 activations with 8 outlier channels x20, "
+        "data": "synthetic (N(0,1) fp16 activations with 8 outlier channels x20, "
                 "uniform int8 weights, random fp16 scales and bias)",
-        "config": {"workload": "configs[1] fused W8A8 linear, M=N=K=4096, fp16 in/out",
+        "config": {"workload": "fused W8A8 linear, M=N=K=4096, fp16 in/out",
                    "M": M, "N": N, "K": K, "parallelism": "single GPU"},
         "roofline": {"bound": "mfma", "achieved": round(achieved, 2), "peak": PEAK_INT8_TOPS,
                      "unit": "TOPS", "frac": round(achieved / PEAK_INT8_TOPS, 4), "traffic": measured_traffic(),

@@ -1,4 +1,4 @@
-// NHWC INT8 conv2d, stride 1, as a window-fed MFMA tile (configs[4]-class shapes: C % 128 == 0,
+// NHWC INT8 conv2d, stride 1, as a window-fed MFMA tile (C % 128 == 0,
 // Co % 256 == 0, a few image rows per tile).
 //
 // The implicit GEMM of the ring-fed tiles (ring_tile.h RingConv) gathers a patch row per output
@@ -8,7 +8,7 @@
 // zeros where it leaves the image) is loaded into LDS once per 128-channel chunk, and every tap's
 // A fragment is read from it at the tap's pixel shift. Only the weights stream per tap
 // (256 rows x 128 bytes a stage: the dense engine's 2-slot ring with a double-buffered window,
-// or, where two windows do not fit, a 3-slot ring with one). For configs[4] (56 x 56 x 256 ->
+// or, where two windows do not fit, a 3-slot ring with one). For 56 x 56 x 256 ->
 // 256, 3x3): 224-pixel tiles move 89 KB of window + 576 KB of weights instead of 2 x 590 KB.
 //
 // Integer sums do not depend on the order of K, so the INT32 result equals the reference's
@@ -346,7 +346,7 @@ int launch_conv_window(const ConvGeom& g, const int8_t* w, const GemmEpilogue& e
     const long long WR = R + static_cast<long long>(kH - 1) * g.dilH;
     const long long nwin = WR * WC;
     const long long nqw = (nwin * 8 + 4 * kWave - 1) / (4 * kWave);
-    // 2 ring slots + two window buffers where they fit (measured faster on configs[4]), else
+    // 2 ring slots + two window buffers where they fit (measured faster at 56 x 56 x 256), else
     // 3 slots + one window buffer.
     const int slots = 2 * 256 * kBK + 2 * nqw * 4 * 1024 <= kWinLds ? 2 : 3;
     const long long lds = static_cast<long long>(slots) * 256 * kBK + (4 - slots) * nqw * 4 * 1024;

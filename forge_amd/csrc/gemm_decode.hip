@@ -1,7 +1,7 @@
 // Decode-shape (M <= 16 tokens) INT8 GEMMs for gfx950, dense and 2:4 sparse: weight
 // streaming at HBM rate.
 //
-// Reference shapes: configs[3] of the reference's decode use (sparse_int8_linear / int8_linear
+// Reference shapes: the reference's decode use (sparse_int8_linear / int8_linear
 // with a handful of tokens, src/gemm/int8_sparse.cu:1005-1043, src/gemm/int8_dense.cu:213-232),
 // where the weights are read once per call and every other operand is tiny.
 //

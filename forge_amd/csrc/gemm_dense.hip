@@ -1,5 +1,6 @@
-// Dense INT8 GEMM for gfx950: C = A (M,K) x B (N,K)^T with exact INT32 accumulation on
-// v_mfma_i32_32x32x32_i8, and the fused dequant + bias epilogue to FP16.
+// Dense INT8 GEMM for gfx950: C = A (M,K) x B (N,K)^T with exact INT32 accumulation on the matrix
+// cores, and the fused dequant + bias epilogue to FP16. This file chooses the engine and holds the
+// register-staged one (v_mfma_i32_32x32x32_i8; the ring-fed tiles use v_mfma_i32_16x16x64_i8).
 //
 // Reference: src/gemm/int8_dense.cu:26-232 (wmma 16x16x16, 128x64 / 128x128 tiles,
 // unpipelined global->smem loads) and src/gemm/int8_gemm.cu:12-46 (dispatch). The

@@ -783,7 +783,7 @@ static int launch_sparse_dma32_tile(const int8_t* W, const int8_t* X, const uint
 
 // The tail split in one launch: workgroups [0, n1) run the whole waves as 256 x 256 tiles over
 // the first nb1 weight blocks, the rest the remaining weight blocks as one wave of 192-token
-// tiles. configs[2] (4096 x 11008 x 4096): 688 tiles on 256 CUs are 2.69 waves, of which the
+// tiles. 4096 x 11008 x 4096: 688 tiles on 256 CUs are 2.69 waves, of which the
 // third runs 69 % full; as 512 tiles + 242 tiles of 192 tokens it takes 2 + ~0.85 tile times.
 template <bool DEQUANT, int BMT2, template <int> class TileT>
 __global__ __launch_bounds__(256) void sparse_dma32_tail_kernel(const int8_t* __restrict__ W,
@@ -841,7 +841,7 @@ static int launch_sparse_dma32_tail(const int8_t* W, const int8_t* X, const uint
 }
 
 // 256 x 256 SMFMAC engine: 256-deep weight stages (full 128-byte lines) for INT32 outputs when
-// K % 256 == 0 (configs[2]: 175 -> 160 us, measured in one run); the FP16 epilogue's registers
+// K % 256 == 0 (4096 x 11008 x 4096: 175 -> 160 us, measured in one run); the FP16 epilogue's registers
 // do not fit beside them (the kernel spills), so dequantizing outputs keep 128-deep stages.
 template <bool DEQUANT>
 static int launch_sparse_dma32(const int8_t* W, const int8_t* X, const uint32_t* meta, const GemmEpilogue& ep,
@@ -1269,7 +1269,7 @@ static int cu_count_or_default() {
 // workgroups per CU). Each engine's time is modelled from the tiles on the busiest CU (w) and
 // the 128-deep stages (steps), with coefficients fitted on MI355X timings of every engine on 30
 // shapes (the reference sweep at M = 1024 / 4096 / 8192, its narrow layers at M up to 147,456,
-// the engine tests' shapes, configs[2] with FP16 out, deep-K layers at M = 256-2048), in us:
+// the engine tests' shapes, 4096 x 11008 x 4096 with FP16 out, deep-K layers at M = 256-2048), in us:
 //   256 x 256: w (0.88 steps + 10.0)
 //   128 x 128: 0.48 steps + 3.7 for one tile per CU, else ceil(w / 2) (0.71 steps + 5.2)
 //   ring:      steps (0.175 ceil(w / 3) + 0.123 w) + 4.6, only up to one round (w <= 3)
@@ -1277,7 +1277,7 @@ static int cu_count_or_default() {
 // 256 x 128 engine, kept for the reference's forced 256x128 tile, was never the fastest there).
 // Examples (us): 1536x6144 at M = 1024 128x128 13.5 (256x256 19.3, 256x128 15.1); 6144x1536 at
 // M = 1024 ring 24.0 (128x128 32.3); 640x320 at M = 147,456 128x128 53.5 (256x256 71.6);
-// configs[2] on 256x256.
+// 4096 x 11008 x 4096 on 256x256.
 enum class SpEngine { k256x256, k256x128, k128x128, kRing };
 constexpr int kSpRingRows = 64, kSpRingDepth = 4, kSpRingPerCu = 3;
 
@@ -1304,7 +1304,7 @@ static SpEngine sparse_pick_engine(int M, int N, int K, int cu)
 // engines run at the same LDS-DMA byte rate): a 256-token tile of NJ 32-row blocks moves 32 KB
 // of tokens + 2.5 KB per block each 128-deep stage, a 256 x 256 tile 52 KB; the 256 x 256 grid
 // takes whole tile waves, the last one a 192-token tail wave (~0.85 of a tile) where
-// launch_sparse_dma32_tail applies. Measured at configs[2] (4096 x 11008 x 4096): 2 x 11-block
+// launch_sparse_dma32_tail applies. Measured at 4096 x 11008 x 4096: 2 x 11-block
 // tiles 115 us vs 2.85 tile times of 256 x 256 126 us; at exact 256 x 256 waves with 8-block
 // wide tiles (4096 x 8192) the two are level by bytes, so the 256 x 256 engine keeps them.
 static bool sparse_wide_pays(int M, int N, int cu, const SpWidePlan& p)

@@ -8,8 +8,8 @@
 // compressed weights and 8 KB of index words through the CU: tokens are most of the bytes, and
 // 2:4 sparsity does not touch them. A tile of 256 tokens x W weight rows moves 64 KB + W * 160 B
 // per slice for 256 W outputs; at W = 352 that is 20 % fewer bytes per output (measured: the
-// DMA-only loop of configs[2], 89 -> 71 us). A workgroup's tiles are planned per CU so that every
-// CU gets the same number of 32-row weight blocks (configs[2], 4096 x 11008: 16 CUs per 256-token
+// DMA-only loop of 4096 x 11008 x 4096, 89 -> 71 us). A workgroup's tiles are planned per CU so that every
+// CU gets the same number of 32-row weight blocks (4096 x 11008: 16 CUs per 256-token
 // block, 21 or 22 blocks each, as two tiles of 10 or 11 blocks: two tile times, where 256 x 256
 // tiles need 2.69 (2.85 with their 192-token tail wave)).
 //
@@ -34,7 +34,7 @@
 // slots this stage used take the stage after next.
 //
 // Epilogue: each wave stages 32 tokens x 64 columns at a time in LDS and writes whole 16-byte row
-// units with cached buffer stores (measured on configs[2]: 116 us cached vs 121.5 us with the
+// units with cached buffer stores (4096 x 11008 x 4096: 116 us cached vs 121.5 us with the
 // non-temporal stores of the other engines; direct stores from the accumulator layout write
 // 32-byte pieces of 32 rows per instruction: 125 us cached, 315 us non-temporal).
 #include "common.h"

@@ -73,8 +73,8 @@ __global__ __launch_bounds__(256) void dequantize_weight_t_kernel(const int8_t* 
 // Column sums of g (M, N) fp16 in FP32, over the rows of part blockIdx.y, to partial (parts, N).
 // A thread sums 8 columns (16-byte loads at element alignment; the last group moved back to end
 // with the row, so that it sums some columns once more, to the same value) of every 4th row, four
-// loads in flight. 2048 x 4096: 5 + 3 us with the second kernel, torch's column sum 14.5 (and
-// its 4.7 us fill).
+// loads in flight. 2048 x 4096, kernel times: 8.0 us and 3.5 for the second kernel, torch's
+// column sum 14.6 and the 4.6 us fill that goes with it.
 __global__ __launch_bounds__(256) void column_sum_kernel(const uint16_t* __restrict__ g, float* __restrict__ partial,
                                                          int M, int N, int rows)
 {

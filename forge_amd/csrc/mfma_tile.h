@@ -263,6 +263,9 @@ struct ConvBytes : ConvGeom {
 
 constexpr int kBK = 128;
 
+// 128-byte LDS rows (8 chunks): chunk c of row r at c ^ ((r ^ (r >> 3)) & 7), made for reads of 32 rows x 2
+// chunks (SQ_LDS_BANK_CONFLICT 0.05 per active LDS cycle at 4096^3). The ring tiles' reads of 16 rows x 4
+// chunks are 2-way conflicted under it (0.50); their measured costs include that.
 __device__ __forceinline__ int lds_swz8(int r) { return (r ^ (r >> 3)) & 7; }
 __device__ __forceinline__ int lds_off128(int r, int c) { return r * kBK + ((c ^ lds_swz8(r)) << 4); }
 

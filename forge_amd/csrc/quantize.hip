@@ -101,7 +101,7 @@ __global__ __launch_bounds__(256) void quantize_rows_block_kernel(
 
 // Rows up to K = 4096 at large M: one wavefront per row, 4 rows per workgroup, so a workgroup
 // moves 4 rows, needs no barrier, and the grid is M/4 workgroups instead of M (at M = 147,456,
-// K = 1280 the per-row workgroups ran at 3.6 TB/s; configs[1], 4096 x 4096: 9.3 -> 8.3 us,
+// K = 1280 the per-row workgroups ran at 3.6 TB/s; 4096 x 4096: 9.3 -> 8.3 us,
 // 6.06 TB/s of 50.3 MB). Lane t holds vectors t, t + 64,
 // ... of its row; loads, absmax and quantization as in the kernel above, the absmax reduced
 // within the wave by DPP.

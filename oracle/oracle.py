@@ -74,7 +74,7 @@ def _declare(L: ctypes.CDLL) -> None:
 
 
 def cpu_threads() -> int:
-    """Threads for the oracle's threaded loops: the host's cores, at most 16 (a GPU box's
+    """Threads for the oracle's threaded loops: the host's cores, at most 16 (a host's
     CPU share per GPU)."""
     try:
         n = len(os.sched_getaffinity(0))

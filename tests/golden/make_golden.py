@@ -6,7 +6,7 @@ a brute-force key formulation of the 2:4 selection), so a test comparing the ora
 or the GPU against these files checks them against an independent derivation.
 
 Inputs:
-  c1_gemm      configs[0] of BASELINE.json: A (128,512), B (256,512) int8 in [-127,127]
+  c1_gemm      A (128,512), B (256,512) int8 in [-127,127]
   quantize     hand-built rows: zero row, one nonzero, exact .5 ties at scale 1.0 and 2.0,
                outlier columns, random N(0,1) rows (fp16)
   prune        tie-heavy int8 groups including -128 / 127
@@ -100,7 +100,7 @@ def pack_gfx950_np(words: np.ndarray, N: int, K: int) -> np.ndarray:
 def main() -> None:
     rng = np.random.default_rng(20261201)
 
-    # --- c1 GEMM (configs[0]) ---------------------------------------------------
+    # --- c1 GEMM ---------------------------------------------------
     A = int8_uniform(np.random.default_rng(1), (128, 512))
     B = int8_uniform(np.random.default_rng(2), (256, 512))
     C = (A.astype(np.int64) @ B.astype(np.int64).T).astype(np.int32)

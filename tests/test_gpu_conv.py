@@ -2,7 +2,7 @@
 
 NHWC implicit GEMM: INT32 bit-exact vs the oracle's direct convolution (golden cases from
 torch float64 conv2d, padding / stride / dilation, C % 16 != 0 byte path, the DMA gather for
-C % 128 == 0 at 128- and 256-row tiles, configs[4] at its full spatial size); FP16 dequant bit-exact to the oracle epilogue. NCHW FP16 API
+C % 128 == 0 at 128- and 256-row tiles, (32,56,56,256) x (256,3,3,256) at its full size); FP16 dequant bit-exact to the oracle epilogue. NCHW FP16 API
 (src/nn/int8_conv2d.cu:126-223): bit-exact to the oracle composition im2col -> per-row
 quantize -> GEMM dequant -> NCHW, and within the reference test's float tolerance
 (tests/test_int8_conv2d.cu:166-176) of a float convolution."""
@@ -115,7 +115,7 @@ def test_conv_window(dev, orc, N, H, W, C, Co, k, pad, dil, route):
 
 
 def test_config5_full_size(dev, orc):
-    """configs[4]: NHWC (32,56,56,256) x (256,3,3,256), stride 1, pad 1; every INT32 output of
+    """NHWC (32,56,56,256) x (256,3,3,256), stride 1, pad 1; every INT32 output of
     all 32 images bit-exact against the oracle's direct convolution (threaded), and every FP16
     output of the per-channel dequant + bias epilogue against the oracle's epilogue on it."""
     import torch

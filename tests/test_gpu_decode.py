@@ -6,7 +6,7 @@ Bar: INT32 bit-exact; FP16 bit-exact to the oracle's epilogue. Shapes exercise t
 K split over 8 wavefronts (K = 128: one wave works; K = 1152: 9 stages, uneven slices and
 idle waves), ragged N (not a multiple of the 32-row workgroup tile), M from 1 to 16 (the
 sparse register kernel with K % 256 == 0, the DMA-ring kernel otherwise), and
-configs[3] at full size (M = 16, 4 and 1, N = K = 8192; every output column); narrow N with K
+N = K = 8192 at M = 16, 4 and 1 (every output column); narrow N with K
 split across workgroups (exact INT32 hand-off), repeated and on two streams at once."""
 import numpy as np
 import pytest
@@ -74,7 +74,7 @@ def test_decode_sparse(dev, orc, M, K, N):
 
 @pytest.mark.parametrize("M", [16, 4, 1])
 def test_config4_full_size(dev, orc, M):
-    """configs[3]: M = 1, 4 and 16 tokens, N = K = 8192, dense and 2:4, FP16 tokens quantized
+    """M = 1, 4 and 16 tokens, N = K = 8192, dense and 2:4, FP16 tokens quantized
     per token, dequant + bias. Every output column against the oracle, through the whole
     int8_linear / sparse_int8_linear and through the GEMM alone on the quantized tokens
     (int8_gemm_dequant / sparse_int8_gemm), with poisoned outputs."""

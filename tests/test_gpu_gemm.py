@@ -3,9 +3,9 @@
 Bar: INT32 bit-exact; FP16 bit-exact to the oracle's epilogue fma((float)acc, as*ws, b)
 (and therefore within the 1-ulp budget against the reference's wmma epilogue,
 src/gemm/int8_dense.cu:171-174); int8_linear's quantized activation bit-exact.
-Shapes cover configs[0] (golden), the reference test's shapes (tests/test_int8_dense_gemm.cu:13,
+Shapes cover 128 x 512 x 256 (golden), the reference test's shapes (tests/test_int8_dense_gemm.cu:13,
 tests/test_int8_dp4a_gemm.cu:180-196 incl. K=7 and K=28), ragged edges, every tile
-configuration, the skinny decode kernel, and configs[1] at full size (sampled rows)."""
+configuration, the skinny decode kernel, and 4096^3 at full size (sampled rows)."""
 import numpy as np
 import pytest
 
@@ -87,7 +87,7 @@ def test_int8_linear(dev, orc, M, K, N):
 
 
 def test_config2_full_size(dev, orc):
-    """configs[1]: W8A8 linear 4096^3, outlier channels; every quantized activation, scale and
+    """W8A8 linear 4096^3, outlier channels; every quantized activation, scale and
     FP16 output compared bit-exactly with the oracle (threaded loop); repeat run bit-identical."""
     import torch
     from forge_amd import ops
@@ -163,7 +163,7 @@ def test_gemm_column_tail_split(dev, orc, M, K, N):
     waves of 256 x 256 tiles over the first tile columns, the remaining columns as one wave of
     192-row tiles, in one launch. (1000, 1024, 17900): 280 tiles = 64 columns x 4 + 6 x 6
     (ragged rows and last column); (512, 1024, 35000): 128 x 2 + 9 x 3; (4096, 4096, 11008):
-    configs[2]'s shape, 32 x 16 + 11 x 22. Every INT32 and FP16 output against the oracle."""
+    32 x 16 + 11 x 22. Every INT32 and FP16 output against the oracle."""
     import torch
     from forge_amd import ops
     rng = np.random.default_rng(M + K + N + 3)

@@ -49,7 +49,7 @@ def _replay_check(dev, calls, outputs, replays=4):
 
 
 def test_graph_int8_linear(dev):
-    """configs[1]-style fused linear (quantize + dequantizing GEMM), plus decode shapes; (16, 4096,
+    """The fused linear (quantize + dequantizing GEMM), plus decode shapes; (16, 4096,
     1024) and (40, 8192, 512) split K across workgroups (on the capture's own sum slot)."""
     import torch
     from forge_amd import ops

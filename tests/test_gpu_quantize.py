@@ -64,7 +64,7 @@ def test_twopass_any_block_size(dev, orc, threads):
 
 
 def test_quantize_outlier_rows_and_ties(dev, orc):
-    """configs[1]'s activation statistics (N(0,1), 8 outlier channels x20) at a small M."""
+    """Transformer activation statistics (N(0,1), 8 outlier channels x20) at a small M."""
     from forge_amd import ops
     rng = np.random.default_rng(7)
     M, K = 64, 4096

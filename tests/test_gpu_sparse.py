@@ -194,7 +194,7 @@ def test_sparse_linear_paths(dev, orc, M, K, N):
 
 
 def test_config3_full_size(dev, orc):
-    """configs[2]: W (11008, 4096) pruned 2:4, A (4096, 4096); every INT32 output bit-exact
+    """W (11008, 4096) pruned 2:4, A (4096, 4096); every INT32 output bit-exact
     against the oracle (threaded loop over the decompressed weights)."""
     import torch
     from forge_amd import ops

@@ -32,7 +32,7 @@ def _prep(dev, W):
 WIDE_SHAPES = [
     (1000, 4096, 17904, 1),   # TB 4, tiles of 8 and 9 blocks, ragged tokens, half last block
     (512, 4096, 35008, 1),    # TB 2, 8/9 blocks, half last block
-    (4096, 2048, 11008, 2),   # configs[2]'s N: 21/22 blocks as 11 + 10 / 11 + 11
+    (4096, 2048, 11008, 2),   # N = 11008: 21/22 blocks as 11 + 10 / 11 + 11
     (8192, 512, 7936, 3),     # TB 32, c 8, K = 512 (four stages): 31 blocks as 11 + 10 + 10
     (8192, 512, 11008, 4),    # 43 blocks as 11 + 11 + 11 + 10
     (3000, 4096, 6720, 1),    # TB 12, c 21: 252 CU slots, no XCD grouping; 10 blocks

@@ -4,7 +4,7 @@ forge_quantize_weight_rows (QuantizedLinear.quantize_weight) and forge_prepare_s
 (SparseLinear.from_dense_weight: quantize + 2:4 prune + compress + gfx950 pack in one pass) are
 compared bit-for-bit with the oracle (whose weight quantization is pinned to the reference's own
 torch expression), for fp32 and fp16 weights, odd shapes, ragged 16-row blocks of the packed
-index words, and the configs[2] weight (11008 x 4096); at that size also against the library's
+index words, and the 11008 x 4096 weight; at that size also against the library's
 separate prune_compress_24 + pack_metadata launches (the reference's two-step sequence)."""
 import numpy as np
 import pytest
@@ -49,7 +49,7 @@ def test_prepare_sparse_weight(dev, orc, N, K, f16):
 
 
 def test_prepare_sparse_weight_full_size(dev):
-    """configs[2]'s weight shape: the one-pass prep equals quantize_weight_rows followed by the
+    """An 11008 x 4096 weight: the one-pass prep equals quantize_weight_rows followed by the
     separate prune_compress_24 and pack_metadata launches."""
     import torch
     from forge_amd import ops
